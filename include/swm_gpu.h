@@ -226,14 +226,15 @@ int swm_gpu_avg_read(swm_ctx *c, int32_t avg_id, double *host_out, double *weigh
  * picks it by hand (1: graphs, 0: direct launches, the default).
  * set_sor_check_every makes the fixed-omega SOR test convergence every `every`
  * sweeps (1..64; the reference mode always tests every sweep).
- * set_sor_halo sets the LDS halo of the blocked fixed-omega sweeps in cells:
- * 2K cells for K sweeps per launch (2, 4 or 8; K must divide the cadence),
- * 0 for one launch per colour, -1 (default) for the largest of 4, 2, 1 sweeps
- * that divides the cadence.  The reference mode (test after every sweep) uses
- * K = halo / 2 sweeps per launch, 4 for halo -1 (each launch also keeps the
- * chi and residual of its earlier sweeps, so any of its sweeps can be the one
- * that passes), and one launch per colour for halo 0.  Every halo gives the
- * same chi bit for bit and, in the reference mode, the same sweep count. */
+ * set_sor_halo sets the halo of the blocked sweeps' tiles in cells: 2K cells
+ * for K sweeps per launch (2, 4 or 8; K must divide the cadence), 0 for one
+ * launch per colour, -1 (default) for four sweeps per launch whatever the
+ * cadence (any sweep of a launch can be a tested one and the one that passes).
+ * Grids with an odd extent that is open across its periodic seam take, for -1,
+ * the largest of 4, 2, 1 sweeps that divides the cadence.  The reference mode
+ * (test after every sweep) uses K = halo / 2 sweeps per launch, 4 for halo -1,
+ * and one launch per colour for halo 0.  Every halo gives the same chi bit for
+ * bit and the same sweep count. */
 int swm_gpu_kernel_shape_count(void);
 int swm_gpu_set_kernel_shape(swm_ctx *c, int32_t shape);
 int swm_gpu_tune(swm_ctx *c, int32_t steps, int32_t *best_shape, double *times_ms);
@@ -241,9 +242,11 @@ int swm_gpu_set_launch_mode(swm_ctx *c, int32_t graphs);
 int swm_gpu_launch_mode(const swm_ctx *c, int32_t *graphs, double *ms_direct, double *ms_graph);
 int swm_gpu_set_sor_check_every(swm_ctx *c, int32_t every);
 int swm_gpu_set_sor_halo(swm_ctx *c, int32_t halo);
-/* rows of the blocked sweeps' 64-column LDS tile: 16 (default) or 32 (fewer
- * halo cells per output; not with the 8-cell halo, whose 64x32 tile would
- * exceed 64 KiB of LDS).  Every tile gives the same chi bit for bit. */
+/* rows of the 64-column LDS tile of grids with an odd extent that is open
+ * across its periodic seam: 16 (default) or 32 (fewer halo cells per output;
+ * not with the 8-cell halo, whose 64x32 tile would exceed 64 KiB of LDS).
+ * Other grids choose their tile by their size.  Every tile gives the same chi
+ * bit for bit. */
 int swm_gpu_set_sor_tile_rows(swm_ctx *c, int32_t rows);
 
 /* computeVelocityPotential (src/calc_lib.f90:500-525) without host copies:

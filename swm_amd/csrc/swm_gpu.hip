@@ -21,6 +21,7 @@
 
 #include "swm_gpu.h"
 #include "swm_kernels.h"
+#include "swm_sor.h"
 
 using swm::Dyn;
 using swm::Fld;
@@ -250,8 +251,14 @@ struct swm_ctx {
     long long* sor_iters = nullptr;
     double* sor_norm = nullptr;
     void* sor_buf[2][2] = {};    // [fp32][chi|B]
-    void* sor_alt[2] = {};       // second chi buffer of the blocked sweeps (ping-pong)
-    void* sor_mid[2][3][2] = {}; // reference mode, K sweeps per launch: chi after each of the first K - 1, by launch parity
+    void* sor_alt[2][2] = {};    // the blocked sweeps' other chi buffers (they go round three; one for sor_block)
+    void* sor_rowc[2] = {};      // sor_rows: padded per-row coefficients and c5 pairs in the sweep precision
+    void* sor_c5p[2] = {};
+    uint8_t* sor_code = nullptr; // sor_rows: per-cell codes
+    double* sor_psum = nullptr;  // sor_rows: partial sums, two sets by launch parity
+    bool sor_closed_x = false, sor_closed_y = false;   // no ocean face across the periodic seam
+    std::vector<double> sor_host[4];                   // c1, c3, c4, c5 rows
+    void* sor_mid[2][3][2] = {}; // sor_block, reference mode, K sweeps per launch: chi after each of the first K - 1, by launch parity
     double* sor_partial_mid = nullptr;   // and their partial sums (3 sweeps x two sets by launch parity)
     void* sor_ftab[2][5] = {};   // coefficient tables in the sweep precision
     void* dza = nullptr;
@@ -654,6 +661,13 @@ int build_tables(swm_ctx* c) {
     std::vector<double> c5r(c5.size());   // correctly rounded reciprocals for dvr (1/-0 = -inf)
     for (size_t k = 0; k < c5.size(); ++k) c5r[k] = 1.0 / c5[k];
     c->sor_tab[4] = upload_vec(c, c5r);
+    c->sor_host[0] = c1;
+    c->sor_host[1] = c3;
+    c->sor_host[2] = c4;
+    c->sor_host[3] = c5;
+    c->sor_closed_x = c->sor_closed_y = true;
+    for (int j = 0; j < Ny; ++j) c->sor_closed_x = c->sor_closed_x && !c->hmask[SWM_GRID_U][(size_t)j * c->Nx];
+    for (int i = 0; i < c->Nx; ++i) c->sor_closed_y = c->sor_closed_y && !c->hmask[SWM_GRID_V][i];
     if (!c->dza || !c->sor_tab[0] || !c->sor_tab[1] || !c->sor_tab[2] || !c->sor_tab[3] || !c->sor_tab[4])
         return fail(c, "table upload failed", 3);
     return 0;
@@ -1564,8 +1578,8 @@ int sor_prepare(swm_ctx* c, bool f32, int nblk) {
     if (!c->sor_buf[w][0]) {
         c->sor_buf[w][0] = dalloc(c, bytes);
         c->sor_buf[w][1] = dalloc(c, bytes);
-        c->sor_alt[w] = dalloc(c, bytes);
-        if (!c->sor_buf[w][0] || !c->sor_buf[w][1] || !c->sor_alt[w]) return fail(c, "out of device memory", 3);
+        c->sor_alt[w][0] = dalloc(c, bytes);
+        if (!c->sor_buf[w][0] || !c->sor_buf[w][1] || !c->sor_alt[w][0]) return fail(c, "out of device memory", 3);
     }
     if (!c->sor_ftab[w][0]) {
         const int Ny = c->Ny;
@@ -1597,6 +1611,166 @@ int sor_prepare(swm_ctx* c, bool f32, int nblk) {
         HIPCHK(c, copy_sync(c, c->sor_relax, relax.data(), relax.size() * 8, hipMemcpyHostToDevice));
         c->sor_nrelax = (int)relax.size();
     }
+    return 0;
+}
+
+// Whether the two colours alternate everywhere a sweep couples cells: even
+// extents, or odd ones with no ocean face across their periodic seam (every
+// closed basin).  sor_rows needs it; other grids take sor_block.
+bool sor_regular(const swm_ctx* c) {
+    return (c->Nx % 2 == 0 || c->sor_closed_x) && (c->Ny % 2 == 0 || c->sor_closed_y);
+}
+
+// Buffers and tables of sor_rows, made on first use and kept: the coefficient
+// tables run from row -kSorPad to kSorPast rows past the last (periodic).
+constexpr int kSorPast = 112;
+template <typename T>
+int sor_rows_prepare(swm_ctx* c) {
+    const int w = std::is_same<T, float>::value ? 1 : 0;
+    const int Nx = c->Nx, Ny = c->Ny;
+    if (!c->sor_code) {
+        if (!(c->sor_code = (uint8_t*)dalloc(c, (size_t)c->P * Ny))) return fail(c, "out of device memory", 3);
+        const long n = (long)Nx * Ny;
+        hipLaunchKernelGGL(swm::sor_code_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, Nx, Ny,
+                           c->P, c->mask, c->sor_code);
+        HIPCHK(c, hipGetLastError());
+        // two sets of sums per tile and sweep: the smallest tile is 112 x 16
+        const size_t tiles = (size_t)((Nx + 111) / 112) * ((Ny + 15) / 16);
+        if (!(c->sor_psum = (double*)dalloc(c, 2 * swm::kSorMaxSweeps * tiles * sizeof(double))))
+            return fail(c, "out of device memory", 3);
+    }
+    if (!c->sor_alt[w][1] && !(c->sor_alt[w][1] = dalloc(c, (size_t)c->P * Ny * sizeof(T))))
+        return fail(c, "out of device memory", 3);
+    if (!c->sor_rowc[w]) {
+        const size_t rows = (size_t)Ny + swm::kSorPad + kSorPast;
+        std::vector<T> rc(8 * rows, T(0)), cp(24 * rows);
+        for (size_t q = 0; q < rows; ++q) {
+            const size_t j = (size_t)((((long)q - swm::kSorPad) % Ny + Ny) % Ny);
+            const double* c5 = &c->sor_host[3][12 * j];
+            for (int k = 0; k < 3; ++k) rc[8 * q + k] = (T)c->sor_host[k][j];
+            rc[8 * q + 3] = (T)c5[11];
+            rc[8 * q + 4] = (T)(1.0 / c5[11]);
+            for (int k = 0; k < 12; ++k) {
+                cp[24 * q + 2 * k] = (T)c5[k];
+                cp[24 * q + 2 * k + 1] = (T)(1.0 / c5[k]);
+            }
+        }
+        if (!(c->sor_rowc[w] = dalloc(c, rc.size() * sizeof(T))) || !(c->sor_c5p[w] = dalloc(c, cp.size() * sizeof(T))))
+            return fail(c, "out of device memory", 3);
+        HIPCHK(c, copy_sync(c, c->sor_rowc[w], rc.data(), rc.size() * sizeof(T), hipMemcpyHostToDevice));
+        HIPCHK(c, copy_sync(c, c->sor_c5p[w], cp.data(), cp.size() * sizeof(T), hipMemcpyHostToDevice));
+    }
+    return 0;
+}
+
+// Tile heights of sor_rows (wavefronts x rows each).  A launch's time is its
+// slowest block's, so a grid takes the smallest tile of which every CU gets at
+// most one (32 rows: 10.1 us a launch against 13.2 with 48 and 15.0 with 64 at
+// 720 x 361 FP64; 64 rows: 10.7 against 12.2 and 13.0 at 1201 x 800 FP32);
+// larger grids take 48 rows, of which a CU holds two, so that one loads while
+// the other sweeps (26.2 against 29.7 with 64 rows at 2048 x 1024 FP64).
+int sor_tile_height(const swm_ctx* c, int H) {
+    auto tiles = [&](int hh) {
+        return (long)((c->Nx + 127 - 2 * H) / (128 - 2 * H)) * ((c->Ny + hh - 2 * H - 1) / (hh - 2 * H));
+    };
+    return tiles(32) <= c->num_cu ? 32 : tiles(64) <= c->num_cu ? 64 : 48;
+}
+
+template <typename T>
+void sor_rows_launch(swm_ctx* c, int hh, const swm::SorRowsArgs<T>& a, const void* in, void* out) {
+    const dim3 grid((unsigned)a.ntile + 1);
+    if (hh == 32)
+        hipLaunchKernelGGL((swm::sor_rows<T, 8, 4>), grid, dim3(512), 0, c->stream, a, (const T*)in, (T*)out);
+    else if (hh == 64)
+        hipLaunchKernelGGL((swm::sor_rows<T, 16, 4>), grid, dim3(1024), 0, c->stream, a, (const T*)in, (T*)out);
+    else
+        hipLaunchKernelGGL((swm::sor_rows<T, 8, 6>), grid, dim3(512), 0, c->stream, a, (const T*)in, (T*)out);
+}
+
+// Up to max_sweeps sweeps in launches of K on register tiles (sor_rows).  chi
+// goes round three buffers, so a launch's input outlives the next launch,
+// whose last block runs the tests: when a sweep inside a launch passes, that
+// launch is run again from its input with the sweeps up to it, and no launch
+// has to keep the chi of every sweep.
+template <typename T>
+int sor_rows_sweeps(swm_ctx* c, void* dchi, void* dB, bool ref_mode, double omega, double tol, double bnorm,
+                    int64_t max_sweeps, int every, int K, int* host_done) {
+    if (int rc = sor_rows_prepare<T>(c)) return rc;
+    const int w = std::is_same<T, float>::value ? 1 : 0;
+    const int H = 2 * K, hh = sor_tile_height(c, H);
+    swm::SorRowsArgs<T> a{};
+    a.Nx = c->Nx; a.Ny = c->Ny; a.P = c->P; a.H = H;
+    a.ntx = (c->Nx + 127 - 2 * H) / (128 - 2 * H);
+    a.ntile = a.ntx * ((c->Ny + hh - 2 * H - 1) / (hh - 2 * H));
+    a.dead_x = c->Nx & 1;
+    a.dead_y = c->Ny & 1;
+    a.B = (const T*)dB;
+    a.code = c->sor_code;
+    a.rowc = (const T*)c->sor_rowc[w];
+    a.c5 = (const T*)c->sor_c5p[w];
+    a.relax = ref_mode ? (const double*)c->sor_relax : nullptr;
+    a.nrelax = c->sor_nrelax;
+    a.omega = omega;
+    a.residual_mode = ref_mode ? 0 : 1;
+    a.eps = tol;
+    a.bnorm = bnorm;
+    a.done = c->sor_done;
+    a.iters = c->sor_iters;
+    a.norm_out = c->sor_norm;
+    void* const buf[3] = {dchi, c->sor_alt[w][0], c->sor_alt[w][1]};
+    auto sums = [&](int64_t n) { return c->sor_psum + (size_t)(n & 1) * swm::kSorMaxSweeps * a.ntile; };
+    auto tests = [&](int64_t first, int nsw) {   // bit q: the q-th sweep from `first` on is tested
+        int m = 0;
+        for (int q = 0; q < nsw; ++q)
+            if ((first + q) % every == 0 || first + q == max_sweeps) m |= 1 << q;
+        return m;
+    };
+    // sweeps enqueued between reads of the convergence flag: 32 at first (a
+    // warm-started solve stops early without queueing many idle launches),
+    // doubling up to 256 for long solves (fewer host round trips)
+    int64_t batch = std::max(32, 4 * every);
+    const int64_t batch_max = std::max(256, 4 * every);
+    int64_t l = 1, n = 0;   // next sweep; launches so far
+    while (l <= max_sweeps && !*host_done) {
+        const int64_t lend = std::min<int64_t>(max_sweeps, l + batch - 1);
+        batch = std::min(2 * batch, batch_max);
+        a.prev_test = 0;
+        // a batch ends with a whole launch unless the sweeps do
+        for (; l <= lend && (l + K - 1 <= lend || lend == max_sweeps); l += K, ++n) {
+            a.nsw = (int)std::min<int64_t>(K, max_sweeps - l + 1);
+            a.sweep = (int)l;
+            a.test = tests(l, a.nsw);
+            a.partial = sums(n);
+            a.prev_partial = sums(n + 1);
+            sor_rows_launch<T>(c, hh, a, buf[n % 3], buf[(n + 1) % 3]);
+            a.prev_test = a.test;
+            a.prev_sweep = a.sweep;
+        }
+        if (a.prev_test)   // the last launch's tests
+            hipLaunchKernelGGL(swm::sor_tests_kernel, dim3(1), dim3(256), 0, c->stream, (const double*)sums(n - 1),
+                               a.ntile, a.prev_test, a.prev_sweep, tol, bnorm, a.residual_mode, a.done, a.iters,
+                               a.norm_out);
+        HIPCHK(c, hipGetLastError());
+        HIPCHK(c, copy_sync(c, host_done, c->sor_done, sizeof(int), hipMemcpyDeviceToHost));
+    }
+    int at = (int)(n % 3);
+    if (*host_done) {
+        long long it = 0;
+        HIPCHK(c, copy_sync(c, &it, c->sor_iters, sizeof(it), hipMemcpyDeviceToHost));
+        const int64_t m = (it - 1) / K;   // the launch that holds the sweep
+        const int q = (int)((it - 1) % K);
+        at = (int)((m + 1) % 3);
+        if (q + 1 < K && it != max_sweeps) {
+            HIPCHK(c, hipMemsetAsync(c->sor_done, 0, sizeof(int), c->stream));
+            a.nsw = q + 1;
+            a.sweep = (int)(m * K + 1);
+            a.test = a.prev_test = 0;
+            sor_rows_launch<T>(c, hh, a, buf[m % 3], buf[at]);
+            HIPCHK(c, hipGetLastError());
+        }
+    }
+    if (buf[at] != dchi)   // the result in the caller's buffer
+        HIPCHK(c, hipMemcpyAsync(dchi, buf[at], (size_t)c->P * c->Ny * sizeof(T), hipMemcpyDeviceToDevice, c->stream));
     return 0;
 }
 
@@ -1649,12 +1823,15 @@ template <typename T>
 int sor_sweeps(swm_ctx* c, void* dchi, void* dB, void* const* tabs, bool ref_mode, double omega, double tol,
                       double bnorm, int64_t max_sweeps, int nblk, int* host_done) {
     const int every = ref_mode ? 1 : c->sor_every;   // the reference tests after every sweep
+    *host_done = 0;
+    if (c->sor_blocked && c->sor_halo != 0 && sor_regular(c))
+        return sor_rows_sweeps<T>(c, dchi, dB, ref_mode, omega, tol, bnorm, max_sweeps, every,
+                                  c->sor_halo < 0 ? 4 : c->sor_halo / 2, host_done);
     // sweeps enqueued between reads of the convergence flag: 32 at first (a
     // warm-started solve stops early without queueing many idle launches),
     // doubling up to 256 for long solves (fewer host round trips)
     int64_t batch = std::max(32, 4 * every);
     const int64_t batch_max = std::max(256, 4 * every);
-    *host_done = 0;
     int64_t l = 1;
     // Blocked sweeps, chi alternating between dchi and the second buffer: K = 4
     // or 2 sweeps per launch in fixed-omega mode when the test cadence is a
@@ -1692,7 +1869,7 @@ int sor_sweeps(swm_ctx* c, void* dchi, void* dB, void* const* tabs, bool ref_mod
         // in the buffer of the launch whose sweep passed.
         const int w = std::is_same<T, float>::value ? 1 : 0;
         void* cur = dchi;
-        void* alt = c->sor_alt[w];
+        void* alt = c->sor_alt[w][0];
         const int ntx = (c->Nx + 63) / 64, nb = ntx * ((c->Ny + rows - 1) / rows);
         const int64_t nfull = max_sweeps / K * K;
         int64_t n = 0;
@@ -1731,7 +1908,7 @@ int sor_sweeps(swm_ctx* c, void* dchi, void* dB, void* const* tabs, bool ref_mod
             const int64_t nconv = (it - 1) / K;   // launch n did sweeps n*K+1 .. (n+1)*K
             const int64_t q = (it - 1) % K;       // the passed sweep's place in it
             if (mid && q < K - 1) cur = c->sor_mid[w][q][nconv & 1];
-            else cur = (nconv & 1) ? dchi : c->sor_alt[w];
+            else cur = (nconv & 1) ? dchi : c->sor_alt[w][0];
         }
         if (cur != dchi)   // the result in the caller's buffer
             HIPCHK(c, hipMemcpyAsync(dchi, cur, (size_t)c->P * c->Ny * sizeof(T), hipMemcpyDeviceToDevice,

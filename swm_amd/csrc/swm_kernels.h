@@ -2105,7 +2105,9 @@ __global__ void __launch_bounds__(256) sor_sweep(const SorArgs<T> a) {
 }
 
 // K sweeps in one launch (fixed omega, or the reference's Chebyshev omega per
-// half sweep) on a TX x TY tile held in LDS with a 2K-cell halo (read from
+// half sweep) on a TX x TY tile held in LDS, for the grids that sor_rows
+// (swm_sor.h) does not take: an odd extent with ocean faces across its
+// periodic seam, where the colours do not alternate.  2K-cell halo (read from
 // chi_in, written to chi_out: blocks read their halos while neighbours write).
 // Half sweep hs updates the colour-(hs % 2) cells at least hs + 1 cells inside
 // the staged block, whose dependency cones stay inside it, so the K sweeps give
