@@ -197,6 +197,7 @@ struct swm_ctx {
     int64_t itt_upload = 0;      // itt of the last state hand-over: the other level holds the
                                  // state before the last step only when itt > itt_upload
     uint8_t* mask = nullptr;
+    uint16_t* code = nullptr;    // per-cell codes of the step kernels (swm::CC_*)
     std::vector<int8_t> hmask[4];
     FieldDev fields[F_COUNT];
     void* tab[T_COUNT] = {};
@@ -727,6 +728,16 @@ int write_statics_t(swm_ctx* c) {
     }
     a.dyn_u = (const T*)c->dyn[0].rec;
     a.dyn_v = (const T*)c->dyn[1].rec;
+    a.code = c->code;
+    a.opt = (a.mix ? swm::OPT_MIX : 0) | (a.quad ? swm::OPT_QUAD : 0) | (a.barotropic ? swm::OPT_BARO : 0) |
+            (a.has_tau_scale ? swm::OPT_TAUSC : 0) | (a.has_taux ? swm::OPT_TAUX : 0) |
+            (a.has_tauy ? swm::OPT_TAUY : 0) | (a.has_ox ? swm::OPT_OX : 0) | (a.has_oy ? swm::OPT_OY : 0) |
+            (a.has_oe ? swm::OPT_OE : 0) | (a.carry ? swm::OPT_CARRY : 0) | (a.nstream ? swm::OPT_STREAM : 0) |
+            (a.dyn_u || a.dyn_v ? swm::OPT_DYN : 0);
+    const Fld<T>* full[] = {&a.He, &a.imu, &a.imv, &a.ime, &a.Fxc, &a.Fyc, &a.Fec, &a.taux, &a.tauy,
+                            &a.timpl[0], &a.gC[0], &a.C0[0], &a.timpl[1], &a.gC[1], &a.C0[1]};   // FULL_* order
+    for (int k = 0; k < 15; ++k)
+        if (full[k]->full) a.opt |= swm::FULL_HE << k;
     static_assert(swm::RT_N >= swm::RT_TRC + swm::RT_PER_TRC * kMaxTracers, "rowtab has room for every tracer");
     if (!c->statics && !(c->statics = dalloc(c, sizeof(Statics<T>)))) return fail(c, "out of device memory", 3);
     if (!c->rowtab && !(c->rowtab = dalloc(c, (size_t)c->Ny * swm::RT_N * sizeof(T)))) return fail(c, "out of device memory", 3);
@@ -1237,6 +1248,26 @@ static int create_impl(swm_ctx* c, const swm_desc* d) {
         c->mask = (uint8_t*)dalloc(c, m.size());
         if (!c->mask) return fail(c, "out of device memory", 3);
         HIPCHK(c, copy_sync(c, c->mask, m.data(), m.size(), hipMemcpyHostToDevice));
+        // per-cell codes: the cell's masks and its neighbours'
+        std::vector<uint16_t> cc((size_t)c->Ny * c->P, 0);
+        const int Nx = c->Nx, Ny = c->Ny;
+        for (int j = 0; j < Ny; ++j) {
+            const uint8_t *r = &m[(size_t)j * c->P], *rs = &m[(size_t)(j ? j - 1 : Ny - 1) * c->P],
+                          *rn = &m[(size_t)(j + 1 < Ny ? j + 1 : 0) * c->P];
+            for (int i = 0; i < Nx; ++i) {
+                const int w = i ? i - 1 : Nx - 1, e = i + 1 < Nx ? i + 1 : 0;
+                auto bit = [](uint8_t x, uint8_t oc, int at) { return x & oc ? 1 << at : 0; };
+                cc[(size_t)j * c->P + i] = (uint16_t)(
+                    r[i] | bit(r[w], swm::OC_E, swm::CC_EW) | bit(rs[i], swm::OC_E, swm::CC_ES) |
+                    bit(rs[w], swm::OC_E, swm::CC_ESW) | bit(rs[i], swm::OC_U, swm::CC_US) |
+                    bit(r[w], swm::OC_V, swm::CC_VW) | bit(rn[i], swm::OC_V, swm::CC_VN) |
+                    bit(r[e], swm::OC_U, swm::CC_UE) | bit(r[e], swm::OC_E, swm::CC_EE) |
+                    bit(rn[i], swm::OC_E, swm::CC_EN) | bit(rn[i], swm::OC_H, swm::CC_HN));
+            }
+        }
+        c->code = (uint16_t*)dalloc(c, cc.size() * sizeof(uint16_t));
+        if (!c->code) return fail(c, "out of device memory", 3);
+        HIPCHK(c, copy_sync(c, c->code, cc.data(), cc.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
     }
     const int8_t *mu = c->hmask[1].data(), *mv = c->hmask[2].data(), *me = c->hmask[3].data();
     int rc = 0;

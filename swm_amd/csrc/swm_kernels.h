@@ -37,6 +37,28 @@ __device__ __forceinline__ T fld(const Fld<T>& f, size_t off, int j, bool ocean)
     return f.full ? f.full[off] : f.rows[2 * j + (ocean ? 0 : 1)];
 }
 
+// Option bits of Statics::opt: one scalar load tells a step kernel everything
+// it branches on (a load, a wait and a branch for each option and field cost
+// more than the branch where a grid is a few blocks per CU).
+enum : unsigned {
+    OPT_MIX = 1u << 0, OPT_QUAD = 1u << 1, OPT_BARO = 1u << 2, OPT_TAUSC = 1u << 3, OPT_TAUX = 1u << 4,
+    OPT_TAUY = 1u << 5, OPT_OX = 1u << 6, OPT_OY = 1u << 7, OPT_OE = 1u << 8, OPT_CARRY = 1u << 9,
+    OPT_STREAM = 1u << 10, OPT_DYN = 1u << 11,
+    FULL_HE = 1u << 16, FULL_IMU = 1u << 17, FULL_IMV = 1u << 18, FULL_IME = 1u << 19, FULL_FXC = 1u << 20,
+    FULL_FYC = 1u << 21, FULL_FEC = 1u << 22, FULL_TAUX = 1u << 23, FULL_TAUY = 1u << 24,
+    FULL_TRC = 1u << 25,   // tracer n: timpl, gC, C0 from bit 25 + 3n
+    FULL_ANY = 0x7fff0000u
+};
+
+// Per-cell code: the ocean masks of the cell (OC_* bits 0-3) and of the
+// neighbours whose masks the stencils need, so a thread reads one code where
+// it would read and combine up to nine mask bytes (the corners it lacks are in
+// the codes to its east and north).
+enum : int {
+    CC_EW = 4, CC_ES = 5, CC_ESW = 6, CC_US = 7, CC_VW = 8, CC_VN = 9, CC_UE = 10, CC_EE = 11, CC_EN = 12, CC_HN = 13,
+    CC_OCEAN = 0x3fff
+};
+
 // Packed per-row values that phase 3 of the tile kernels reads, RT_N per row
 // (Statics::rowtab): built on the device from the per-row tables and the
 // row-compressed fields whenever the statics are written.  A field stored as
@@ -60,6 +82,8 @@ struct Statics {
     int mix, quad, barotropic, has_tau_scale;
     int carry;           // FP32 state carries its bfloat16 low part (lo planes read and written)
     int has_taux, has_tauy, has_ox, has_oy, has_oe;
+    unsigned opt;        // OPT_* bits: the options above and which fields are full arrays, in one word
+    const uint16_t* code;   // per-cell masks of the cell and its neighbours (CC_*)
     T G, A, dL, dT, RHO0, minD, lbc, tau_scale, AdT, eps;
     T rdL, rdT, rAdT;    // 1/dL, 1/dT, 1/AdT (correctly rounded, for dvr)
     const uint8_t* mask;
@@ -347,23 +371,23 @@ __device__ __forceinline__ T trc_adv_r(bool neg, int nummask, int den, const T* 
 }
 
 // LDS of one tile: the state with a one-cell halo, the derived fields and the
-// per-row coefficient tables of its rows.  eta shares its array with Pot (each
-// cell reads its own eta before writing its Pot), and the mass fluxes MU, MV
-// are formed from Du, Dv and u, v where they are needed, which keeps the FP64
-// tile under 32 KiB (five blocks per CU).  NTR is the largest tracer count the
+// per-row coefficient tables of its rows.  eta shares its array with EDens
+// (each cell reads its own eta before writing its EDens), and in FP64 the mass
+// fluxes MU, MV are formed from D and u, v where they are needed, which keeps the
+// FP64 tile under 32 KiB (five blocks per CU).  NTR is the largest tracer count the
 // kernel handles.
 template <typename T, int NTR, int E, int EH, int ZE = 1, int DUE = 1, int DVE = 1, int RTR = 1, int RTK_ = 1>
 struct TileLds {
     static constexpr int RTK = RTK_;
-    T u[E], v[E], D[E], Pot[E], Ed[E], pll[E], plt[E];   // Pot holds eta until phase 2 replaces it
+    T u[E], v[E], D[E], Pot[E], Ed[E], pll[E], plt[E];   // D is 0 on land; Ed holds eta until phase 2 replaces it
     T zt[ZE], et[ZE];    // LINEARISED_MEAN_STATE (ZE = E): relative vorticity and eta for phase 3
-    T Du[DUE], Dv[DVE];  // interp2(D, eta2u/eta2v_noland) of every halo cell (when DUE / DVE = E)
-    T CH[NTR][E], C[NTR][E];
+    T Du[DUE], Dv[DVE], MU[DUE], MV[DVE];   // interp2(D, eta2u/eta2v_noland) and the mass fluxes (when DUE / DVE = E)
+    T CH[NTR ? NTR : 1][NTR ? E : 1], C[NTR ? NTR : 1][NTR ? E : 1];
     // per-row tables of the EH tile rows (cu also of the row above them)
     T za[EH][2], cu[EH + 1], cH[EH], rcH[EH], fH[EH], pltc[EH][12], pllc[EH][12];
     T rt[RTR][RTK_];     // rowtab rows of the output rows and the row after them (RowTabC)
     int ocean[4];        // per wavefront: all of its halo cells are ocean at every point (tile_body)
-    uint8_t m[E];
+    uint16_t m[E];       // cell codes
 };
 
 // Phase 3's per-row values: tiles whose wavefronts span several rows stage
@@ -381,11 +405,10 @@ struct RowTabC {
     static constexpr int NQ = UROW ? 1 : (R * K + 255) / 256;
 };
 
-// Tiles that keep Du and Dv in LDS, computed once per halo cell in phase 2
+// Tiles that keep Du, Dv, MU and MV in LDS, computed once per cell in phase 2
 // instead of at each stencil point in phase 3: the FP32 tiles, which have
-// LDS to spare at their occupancy (measured 0.8 % faster at 1024^2).  FP64
-// recomputes them (no faster with Du kept, and the 64-wide tiles would drop
-// to four blocks per CU).
+// LDS to spare at their occupancy.  FP64 recomputes them (its tiles would drop
+// to three or four blocks per CU).
 template <typename T, int TX, int TY>
 struct LdsDuDv {
     static constexpr int E = (TX + 2) * (TY + 2);
@@ -439,11 +462,13 @@ __device__ __forceinline__ void apply_streams(S& a, const Dyn<T>& d, size_t off,
         if (!d.ss[n].exact) y = y0 + dv(d.ss[n].a * (gld(r + d.ss[n].o1, off) - y0), d.ss[n].b);
         if (a.skind[n] == 0) {
             const T num = a.has_tau_scale ? a.tau_scale * y : y;
-            y = a.sdiv ? dv(num, a.RHO0 * (comp == 0 ? Du : Dv)) : dv(num, a.RHO0);
+            y = dv(num, a.sdiv ? a.RHO0 * (comp == 0 ? T(Du) : T(Dv)) : a.RHO0);
         }
-        if (comp == 0) Fx = Fx + y;
-        else if (comp == 1) Fy = Fy + y;
-        else Fe = Fe + y;
+        // selects, not stores through the references: the three sums stay in registers
+        const T x0 = Fx + y, x1 = Fy + y, x2 = Fe + y;
+        Fx = comp == 0 ? x0 : Fx;
+        Fy = comp == 1 ? x1 : Fy;
+        Fe = comp == 2 ? x2 : Fe;
     }
 }
 
@@ -455,7 +480,7 @@ struct TileRegs {
     T rt[NQ];    // rowtab values for the LDS row table (RowTabC)
     int m[NE];
     int ocean;   // every halo cell of this thread is ocean at all four points
-    T u[NE], v[NE], e[NE], Ho[NE], Hl[NE], ch[NTR][NE], cb[NTR][NE];
+    T u[NE], v[NE], e[NE], H[NE], ch[NTR][NE], cb[NTR][NE];
     T tz0, tz1, tcu, tcH, tfH, tcu0, tpc;
     T g[NO][6];
     T gt[NO][NTR][2];
@@ -472,12 +497,11 @@ struct TileShapeC {
 // Issue the loads of the outputs' AB history (2 slots per field and tracer)
 // and eta at the outputs into R.
 template <typename T, int VAR, int NTRC, int TX, int TY, bool DIAG, typename RG>
-__device__ __forceinline__ void tile_load_hist(const Dyn<T>& d, const int t, RG& R) {
+__device__ __forceinline__ void tile_load_hist(const Dyn<T>& d, const int t, RG& R, const int tid) {
     if (DIAG) return;
     constexpr int NT = 256;
     constexpr int NO = (TX * TY + NT - 1) / NT;
     CStatics<T>& a = *(CStatics<T>*)d.s;
-    const int tid = threadIdx.x;
     const int i0 = (t % d.ntx) * TX;
     const int j0 = (t / d.ntx) * TY;
     const int Nx = a.Nx, Ny = a.Ny, P = a.P;
@@ -512,7 +536,7 @@ __device__ __forceinline__ void tile_load_hist(const Dyn<T>& d, const int t, RG&
                     pt[q][n][1] = gld(tb, r1 * pl + off);
                 }
                 if constexpr (sizeof(T) == 4) {
-                    if (a.carry) {
+                    if (a.opt & OPT_CARRY) {
 #pragma unroll
                         for (int f = 0; f < 3; ++f) R.lo[q][f] = gld(lo_plane(st, pl, PL_LO + f), off);
 #pragma unroll
@@ -532,7 +556,7 @@ __device__ __forceinline__ void tile_load_hist(const Dyn<T>& d, const int t, RG&
 // Issue every global load of tile t: the state with its halo, the per-row
 // tables and the AB history of the outputs.
 template <typename T, int VAR, int NTRC, int TX, int TY, bool DIAG, bool HIST = true, typename RG>
-__device__ __forceinline__ void tile_load(const Dyn<T>& d, const int t, RG& R) {
+__device__ __forceinline__ void tile_load(const Dyn<T>& d, const int t, RG& R, const int tid) {
     constexpr int NT = 256;
     constexpr int EW = TX + 2;
     constexpr int EH = TY + 2;
@@ -540,7 +564,6 @@ __device__ __forceinline__ void tile_load(const Dyn<T>& d, const int t, RG& R) {
     constexpr int NO = (TX * TY + NT - 1) / NT;
     constexpr int NTR = NTRC > 0 ? NTRC : 1;
     CStatics<T>& a = *(CStatics<T>*)d.s;
-    const int tid = threadIdx.x;
     const int i0 = (t % d.ntx) * TX;
     const int j0 = (t / d.ntx) * TY;
     const int Nx = a.Nx, Ny = a.Ny, P = a.P;
@@ -559,7 +582,7 @@ __device__ __forceinline__ void tile_load(const Dyn<T>& d, const int t, RG& R) {
     const T* const Ge1 = st + (PL_GE + r0) * pl;
     const T* const Ge2 = st + (PL_GE + r1) * pl;
 
-    if (HIST) tile_load_hist<T, VAR, NTRC, TX, TY, DIAG>(d, t, R);
+    if (HIST) tile_load_hist<T, VAR, NTRC, TX, TY, DIAG>(d, t, R, tid);
 
     // tiles no larger than the grid: every halo and table index is within one
     // period of it
@@ -572,11 +595,12 @@ __device__ __forceinline__ void tile_load(const Dyn<T>& d, const int t, RG& R) {
     auto& ru = R.u;
     auto& rv = R.v;
     auto& re = R.e;
-    auto& rHo = R.Ho;
-    auto& rHl = R.Hl;
+    auto& rH = R.H;
     auto& rch = R.ch;
     auto& rcb = R.cb;
     R.ocean = 1;
+    const unsigned opt = a.opt;
+    const bool hef = (opt & FULL_HE) != 0;
 #pragma unroll
     for (int q = 0; q < NE; ++q) {
         const int e = tid + q * NT;
@@ -591,14 +615,12 @@ __device__ __forceinline__ void tile_load(const Dyn<T>& d, const int t, RG& R) {
                 gj = wrap(gj, Ny);
             }
             const size_t off = (size_t)gj * P + gi;
-            rm[q] = gld(a.mask, off);
-            R.ocean &= rm[q] == 15;
+            rm[q] = gld(a.code, off);
+            R.ocean &= (rm[q] & 15) == 15;
             ru[q] = gld(su, off);
             rv[q] = gld(sv, off);
             re[q] = gld(se, off);
-            // H_eta at an ocean (rHo) and a land (rHl) point of this cell's row
-            rHo[q] = a.He.full ? gld(a.He.full, off) : gld(a.He.rows, 2 * (size_t)gj);
-            rHl[q] = a.He.full ? rHo[q] : gld(a.He.rows, 2 * (size_t)gj + 1);
+            rH[q] = hef ? gld(a.He.full, off) : gld(a.He.rows, 2 * (size_t)gj);   // read on ocean points only
 #pragma unroll
             for (int n = 0; n < NTRC; ++n) {
                 const T* tb = st + (PL_TRC + PL_PER_TRC * n) * pl;
@@ -624,7 +646,7 @@ __device__ __forceinline__ void tile_load(const Dyn<T>& d, const int t, RG& R) {
         tfH = gld(a.fH, gj);
     }
     if (tid == NT - 1) tcu0 = gld(a.cu, wrap(j0 - 2, Ny));
-    const bool has_pc = a.mix && tid < EH * 24;
+    const bool has_pc = (opt & OPT_MIX) && tid < EH * 24;
     if (has_pc) {
         const int r = tid / 24, c = tid % 24;
         const int gj = wrap(j0 + r - 1, Ny);
@@ -645,7 +667,7 @@ __device__ __forceinline__ void tile_load(const Dyn<T>& d, const int t, RG& R) {
 
 // Derive D and C from the loaded state and write the tile to LDS.
 template <typename T, int VAR, int NTRC, int TX, int TY, bool DIAG, typename RG, typename L>
-__device__ __forceinline__ void tile_stage(const Dyn<T>& d, const int t, const RG& R, L& lds) {
+__device__ __forceinline__ void tile_stage(const Dyn<T>& d, const int t, const RG& R, L& lds, const int tid) {
     constexpr int NT = 256;
     constexpr int EW = TX + 2;
     constexpr int EH = TY + 2;
@@ -654,18 +676,13 @@ __device__ __forceinline__ void tile_stage(const Dyn<T>& d, const int t, const R
     constexpr int NTR = NTRC > 0 ? NTRC : 1;
     T* const s_u = lds.u;
     T* const s_v = lds.v;
-    T* const s_eta = lds.Pot;
+    T* const s_eta = lds.Ed;
     T* const s_D = lds.D;
-    T* const s_Pot = lds.Pot;
-    T* const s_Ed = lds.Ed;
-    T* const s_pll = lds.pll;
-    T* const s_plt = lds.plt;
     auto& s_CH = lds.CH;
     auto& s_C = lds.C;
-    uint8_t* const s_m = lds.m;
+    uint16_t* const s_m = lds.m;
 
     CStatics<T>& a = *(CStatics<T>*)d.s;
-    const int tid = threadIdx.x;
     const int i0 = (t % d.ntx) * TX;
     const int j0 = (t / d.ntx) * TY;
     const int Nx = a.Nx, Ny = a.Ny, P = a.P;
@@ -689,28 +706,27 @@ __device__ __forceinline__ void tile_stage(const Dyn<T>& d, const int t, const R
     const auto& ru = R.u;
     const auto& rv = R.v;
     const auto& re = R.e;
-    const auto& rHo = R.Ho;
-    const auto& rHl = R.Hl;
+    const auto& rH = R.H;
     const auto& rch = R.ch;
     const auto& rcb = R.cb;
     const T tz0 = R.tz0, tz1 = R.tz1, tcu = R.tcu, tcH = R.tcH, tfH = R.tfH, tcu0 = R.tcu0, tpc = R.tpc;
-    const bool has_pc = a.mix && tid < EH * 24;
+    const bool mix = (a.opt & OPT_MIX) != 0, has_pc = mix && tid < EH * 24;
 #pragma unroll
     for (int q = 0; q < NE; ++q) {
         const int e = tid + q * NT;
         if (e < E) {
             const int m = rm[q];
             const T eta = re[q];
-            s_m[e] = (uint8_t)m;
+            s_m[e] = (uint16_t)m;
             s_u[e] = ru[q];
             s_v[e] = rv[q];
             s_eta[e] = eta;
             if constexpr (VAR == VAR_MS) lds.et[e] = eta;
-            const T He = OE(m) ? rHo[q] : rHl[q];
-            T D;
-            if (FN) D = OE(m) ? (eta + He) : T(1);   // computeD: D = eta + H on ocean eta, 1 elsewhere
-            else D = He;                              // linear variants: D aliases H_eta
-            s_D[e] = D;
+            // computeD: D = eta + H on ocean eta, 1 elsewhere; the linear variants
+            // alias H_eta.  LDS holds 0 on land, which the interpolations weight by 0.
+            const T Do = FN ? eta + rH[q] : rH[q];
+            const T D = OE(m) ? Do : T(1);
+            s_D[e] = OE(m) ? Do : T(0);
 #pragma unroll
             for (int n = 0; n < NTRC; ++n) {
                 s_CH[n][e] = rch[n][q];
@@ -733,7 +749,7 @@ __device__ __forceinline__ void tile_stage(const Dyn<T>& d, const int t, const R
         if (c < 12) lds.pltc[r][c] = tpc;
         else lds.pllc[r][c - 12] = tpc;
     }
-    if (EH * 24 > NT && a.mix)   // tiles taller than 8 rows: the remaining table rows
+    if (EH * 24 > NT && mix)   // tiles taller than 8 rows: the remaining table rows
         for (int q = tid + NT; q < EH * 24; q += NT) {
             const int r = q / 24, c = q % 24;
             const int gj = wrap(j0 + r - 1, Ny);
@@ -753,23 +769,27 @@ __device__ __forceinline__ void tile_stage(const Dyn<T>& d, const int t, const R
 // Phases 2 and 3 of tile t, after its LDS stage and a barrier: derived fields,
 // tendencies, AB integration and stores.  pg/pt: the outputs' AB history.
 // OCEAN: every cell of the tile and of its halo is ocean at its u, v, eta and
-// H points.  The masks are then the constant 15 and the mask arithmetic
-// (no-land weights, land selects, coefficient rows) folds away at compile
-// time; the expressions left are the general path's with every mask 1, so
-// both give the same bits on such a tile.
+// H points.  The masks are then constants and the mask arithmetic (no-land
+// weights, land selects, coefficient rows) folds away at compile time; the
+// expressions left are the general path's with every mask 1, so both give the
+// same bits on such a tile.
+//
+// Neither phase branches on a mask: every lane forms every term and land takes
+// its value by a select, so a phase is a few straight runs of code whose LDS
+// reads are issued together.  With a branch around each masked term (62 of
+// them in the FP64 kernel with a tracer) each waited for its own LDS reads and
+// the phases took 13 000 cycles of a block that had its CU to itself, three
+// times their issue time.
 template <typename T, int VAR, int NTRC, int TX, int TY, bool DIAG, bool DYN = true, bool OCEAN = false, typename L,
           typename G, typename GT, typename GE, typename LO>
 __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& lds, const G& pg, const GT& pt,
-                                             const GE& pe, const LO& plo) {
+                                             const GE& pe, const LO& plo, const int tid) {
     constexpr int NT = 256;
     constexpr int EW = TX + 2;
-    constexpr int EH = TY + 2;
-    constexpr int E = EW * EH;
     constexpr int NO = (TX * TY + NT - 1) / NT;
-    constexpr int NTR = NTRC > 0 ? NTRC : 1;
     T* const s_u = lds.u;
     T* const s_v = lds.v;
-    T* const s_eta = lds.Pot;
+    T* const s_eta = lds.Ed;
     T* const s_D = lds.D;
     T* const s_Pot = lds.Pot;
     T* const s_Ed = lds.Ed;
@@ -777,212 +797,131 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
     T* const s_plt = lds.plt;
     auto& s_CH = lds.CH;
     auto& s_C = lds.C;
-    const uint8_t* const s_m = lds.m;
-    // mask byte of LDS cell e
-    auto M = [&](int e) -> uint8_t {
-        if constexpr (OCEAN) return 15;
+    const uint16_t* const s_m = lds.m;
+    // code of LDS cell e
+    auto M = [&](int e) -> int {
+        if constexpr (OCEAN) return CC_OCEAN;
         else return s_m[e];
     };
+    auto B = [](int code, int at) -> bool { return ((code >> at) & 1) != 0; };
 
     CStatics<T>& a = *(CStatics<T>*)d.s;
-    const int tid = threadIdx.x;
+    const unsigned opt = a.opt;
     const int i0 = (t % d.ntx) * TX;
     const int j0 = (t / d.ntx) * TY;
     const int Nx = a.Nx, Ny = a.Ny, P = a.P;
-    const bool FN = (VAR == VAR_FN);
+    constexpr bool FN = VAR == VAR_FN;
     // planes of this step's roles
     T* const st = d.state;
     const long long pl = d.plane;
-    const int r0 = d.ring, r1 = d.ring == 2 ? 0 : d.ring + 1, r2 = d.ring == 0 ? 2 : d.ring - 1;
-    const T* const su = st + (PL_U + d.cur) * pl;
-    const T* const sv = st + (PL_V + d.cur) * pl;
+    const int r2 = d.ring == 0 ? 2 : d.ring - 1;
     const T* const se = st + (PL_E + d.cur) * pl;
-    const T* const Gu1 = st + (PL_GU + r0) * pl;
-    const T* const Gu2 = st + (PL_GU + r1) * pl;
-    const T* const Gv1 = st + (PL_GV + r0) * pl;
-    const T* const Gv2 = st + (PL_GV + r1) * pl;
-    const T* const Ge1 = st + (PL_GE + r0) * pl;
-    const T* const Ge2 = st + (PL_GE + r1) * pl;
+    constexpr bool SDU = LdsDuDv<T, TX, TY>::SDU, SDV = LdsDuDv<T, TX, TY>::SDV;
+    // interp2(D, eta2u/eta2v_noland) of two cells of D (0 on land): each takes
+    // half where both are ocean, else the ocean one is the whole
+    auto mid = [](T D1, T D2, bool both) -> T {
+        const T w = both ? T(0.5) : T(1);
+        return fm(w, D2, w * D1);
+    };
 
-    // ---- phase 2: derived fields on the extended tile
-    constexpr bool SPLIT2 = !DIAG && !LdsDuDv<T, TX, TY>::SDU && !LdsDuDv<T, TX, TY>::SDV;
-    if constexpr (SPLIT2) {
-        // Two loops over the two regions the stencils need, instead of one loop
-        // over the whole (TX+2)(TY+2) tile: EDens and P_lambda-lambda on
-        // lx 0..TX, ly 0..TY, then (Pot overwrites eta in place) Dh, zeta, Pot
-        // and P_lambda-theta on lx 1..TX+1, ly 1..TY+1.  Each has
-        // (TX+1)(TY+1) cells; their second passes run on different waves
-        // (tid ^ 128: wave 2 for the first loop, wave 0 for the second; wave 3
-        // for the second measured 0.5 % slower).
-        constexpr int RW = TX + 1, NR = (TX + 1) * (TY + 1);
-        for (int r = tid ^ 128; r < NR; r += NT) {
-            const int lx = r % RW, ly = r / RW;
-            const int e = ly * EW + lx;
-            const uint8_t m = M(e);
-            const int ke = e + 1, kn = e + EW;
-            T Ed = T(0);
-            if (OE(m)) {
-                if (FN) {
-                    const T ue = s_u[ke], uc = s_u[e], vn = s_v[kn], vc = s_v[e];
-                    Ed = fm(a.G, s_eta[e],
-                            (fm(T(0.5), uc * uc, T(0.5) * (ue * ue)) + fm(T(0.5), vc * vc, T(0.5) * (vn * vn))) / T(2));
-                } else if (VAR == VAR_MS) {   // g*eta + uU + vV
-                    const int gj = wrap(j0 + ly - 1, Ny);
-                    const int gi = wrap(i0 + lx - 1, Nx), gip = gi + 1 == Nx ? 0 : gi + 1;
-                    const int gjp = gj + 1 == Ny ? 0 : gj + 1;
-                    const T ube = fldg(a.ubs, (size_t)gj * P + gip, gj, OU(M(ke)) != 0);
-                    const T ubc = fldg(a.ubs, (size_t)gj * P + gi, gj, OU(m) != 0);
-                    const T vbn = fldg(a.vbs, (size_t)gjp * P + gi, gjp, OV(M(kn)) != 0);
-                    const T vbc = fldg(a.vbs, (size_t)gj * P + gi, gj, OV(m) != 0);
-                    const T ue = s_u[ke], uc = s_u[e], vn = s_v[kn], vc = s_v[e];
-                    Ed = ((T(0.5) * (ue * ube) + T(0.5) * (uc * ubc)) + (T(0.5) * (vn * vbn) + T(0.5) * (vc * vbc))) +
-                         a.G * s_eta[e];
-                } else {
-                    Ed = a.G * s_eta[e];
-                }
-            }
-            s_Ed[e] = Ed;
-            T pll = T(0);
-            if (a.mix && OE(m)) {
-                const T* c = &lds.pllc[ly][(OV(M(kn)) * 2 + OV(m)) * 3];
-                pll = s_D[e] * fm(c[2], s_v[e], fm(c[1], s_v[kn], c[0] * (s_u[ke] - s_u[e])));
-            }
-            s_pll[e] = pll;
+    // ---- phase 2: derived fields.  Every field is needed on (TX+1)(TY+1)
+    // cells of the halo tile, each on its own corner of it: task r takes the
+    // 2 x 2 cells whose south-west one is A and forms EDens and
+    // P_lambda-lambda at A, Dh, zeta, Pot and P_lambda-theta at the
+    // north-east cell Q, and in FP32 Du, MU at the south-east cell and Dv, MV
+    // at the north-west one.
+    constexpr int RW = TX + 1, NR = (TX + 1) * (TY + 1);
+    for (int r = tid; r < NR; r += NT) {
+        const int lx = r % RW, ly = r / RW;
+        const int A = ly * EW + lx, Es = A + 1, Nw = A + EW, Q = Nw + 1;
+        const int ca = M(A), cq = M(Q);
+        const bool oe = B(ca, 3);
+        const T ua = s_u[A], ub = s_u[Es], ud = s_u[Q], va = s_v[A], vc = s_v[Nw], vd = s_v[Q];
+        const T Da = s_D[A], Db = s_D[Es], Dc = s_D[Nw], Dd = s_D[Q];
+        const T eta = s_eta[A];
+        // computeEdens (src/swm_timestep_module.f90:259-310); land keeps 0
+        T Ed;
+        if (FN) {
+            Ed = fm(a.G, eta, (fm(T(0.5), ua * ua, T(0.5) * (ub * ub)) + fm(T(0.5), va * va, T(0.5) * (vc * vc))) / T(2));
+        } else if (VAR == VAR_MS) {   // g*eta + uU + vV
+            const int gj = wrap(j0 + ly - 1, Ny), gjp = gj + 1 == Ny ? 0 : gj + 1;
+            const int gi = wrap(i0 + lx - 1, Nx), gip = gi + 1 == Nx ? 0 : gi + 1;
+            const T ube = fldg(a.ubs, (size_t)gj * P + gip, gj, OU(M(Es)) != 0);
+            const T ubc = fldg(a.ubs, (size_t)gj * P + gi, gj, OU(ca) != 0);
+            const T vbn = fldg(a.vbs, (size_t)gjp * P + gi, gjp, OV(M(Nw)) != 0);
+            const T vbc = fldg(a.vbs, (size_t)gj * P + gi, gj, OV(ca) != 0);
+            Ed = ((T(0.5) * (ub * ube) + T(0.5) * (ua * ubc)) + (T(0.5) * (vc * vbn) + T(0.5) * (va * vbc))) + a.G * eta;
+        } else {
+            Ed = a.G * eta;
         }
-        __syncthreads();   // every eta read before Pot takes its place
-        for (int r = tid; r < NR; r += NT) {
-            const int lx = r % RW + 1, ly = r / RW + 1;
-            const int e = ly * EW + lx;
-            const int gj = wrap(j0 + ly - 1, Ny);
-            const uint8_t m = M(e);
-            const int kw = e - 1, ks = e - EW, ksw = e - EW - 1;
-            const int m1 = OE(m), m2 = OE(M(ksw)), m3 = OE(M(kw)), m4 = OE(M(ks));
-            const T w = noland_w<T>(m1 + m2 + m3 + m4);
-            const T Dh = fm(m4 ? w : T(0), s_D[ks],
-                            fm(m3 ? w : T(0), s_D[kw], fm(m2 ? w : T(0), s_D[ksw], (m1 ? w : T(0)) * s_D[e])));
-            T zeta = T(0);
-            if (FN || VAR == VAR_MS) {
-                T za_ = T(0), zb = T(0);
-                if (OV(M(kw)) + OV(m) != 0)
-                    za_ = lds.za[ly][OH(m) ? 0 : 1] * (s_v[e] - s_v[kw]);
-                if (OU(m) + OU(M(ks)) != 0) {
-                    const T bcH = OH(m) ? T(1) : a.lbc;
-                    zb = dvr(bcH * fm(-lds.cu[ly], s_u[ks], lds.cu[ly + 1] * s_u[e]), a.AdT, a.rAdT);
-                }
-                zeta = za_ - dvr(zb, lds.cH[ly], lds.rcH[ly]);
-            }
-            const T pD = Dh > a.eps ? Dh : a.eps;
-            T Pot;
-            if constexpr (VAR == VAR_MS) {   // (f + zeta_bs) / pD
-                const int gi = wrap(i0 + lx - 1, Nx);
-                Pot = dv(lds.fH[ly] + fldg(a.zbs, (size_t)gj * P + gi, gj, OH(m)), pD);
-                lds.zt[e] = zeta;
-            } else {
-                Pot = FN ? dv(lds.fH[ly] + zeta, pD) : dv(lds.fH[ly], pD);
-            }
-            s_Pot[e] = Pot;
-            T plt = T(0);
-            if (a.mix && OH(m)) {
-                const T* c = &lds.pltc[ly][(OU(m) * 2 + OU(M(ks))) * 3];
-                plt = Dh * fm(c[2], s_u[ks], fm(c[1], s_u[e], c[0] * (s_v[e] - s_v[kw])));
-            }
-            s_plt[e] = plt;
+        s_Ed[A] = oe ? Ed : T(0);
+        // Dh = interp4(D, eta2H_noland): points (i,j), (i-1,j-1), (i-1,j), (i,j-1)
+        const int n4 = OE(cq) + OE(ca) + ((cq >> CC_EW) & 1) + ((cq >> CC_ES) & 1);
+        const T w4 = noland_w<T>(n4);
+        const T Dh = fm(w4, Db, fm(w4, Dc, fm(w4, Da, w4 * Dd)));
+        // computeRelVort -> vorticityFromVelocities2D (src/calc_lib.f90:663-678,
+        // pder_zonal3D 892-926, pder_meridional3D 965-998)
+        const bool oh = B(cq, 0);
+        T zeta = T(0);
+        if (FN || VAR == VAR_MS) {
+            const T z1 = lds.za[ly + 1][oh ? 0 : 1] * (vd - vc);
+            const T za_ = (OV(cq) | ((cq >> CC_VW) & 1)) ? z1 : T(0);
+            const T bcH = oh ? T(1) : a.lbc;
+            const T z2 = dvr(bcH * fm(-lds.cu[ly + 1], ub, lds.cu[ly + 2] * ud), a.AdT, a.rAdT);
+            const T zb = (OU(cq) | ((cq >> CC_US) & 1)) ? z2 : T(0);
+            zeta = za_ - dvr(zb, lds.cH[ly + 1], lds.rcH[ly + 1]);
         }
-    } else
-    for (int e = tid; e < E; e += NT) {
-        const int lx = e % EW, ly = e / EW;
-        const int gj = wrap(j0 + ly - 1, Ny);
-        const uint8_t m = M(e);
-        const bool interior = DIAG && lx >= 1 && lx <= TX && ly >= 1 && ly <= TY &&
-                              (i0 + lx - 1) < Nx && (j0 + ly - 1) < Ny;
-        const size_t doff = interior ? (size_t)(j0 + ly - 1) * P + (i0 + lx - 1) : 0;
-        const T eta_e = s_eta[e];   // before this cell's Pot takes its place
-        if (lx >= 1 && ly >= 1) {
-            const int kw = e - 1, ks = e - EW, ksw = e - EW - 1;
-            // Dh = interp4(D, eta2H_noland): points (i,j), (i-1,j-1), (i-1,j), (i,j-1)
-            const int m1 = OE(m), m2 = OE(M(ksw)), m3 = OE(M(kw)), m4 = OE(M(ks));
-            const T w = noland_w<T>(m1 + m2 + m3 + m4);
-            const T Dh = fm(m4 ? w : T(0), s_D[ks],
-                            fm(m3 ? w : T(0), s_D[kw], fm(m2 ? w : T(0), s_D[ksw], (m1 ? w : T(0)) * s_D[e])));
-            // computeRelVort -> vorticityFromVelocities2D (src/calc_lib.f90:663-678,
-            // pder_zonal3D 892-926, pder_meridional3D 965-998)
-            T zeta = T(0);
-            if (FN || VAR == VAR_MS) {
-                const int gjm = gj == 0 ? Ny - 1 : gj - 1;
-                T za_ = T(0), zb = T(0);
-                if (OV(M(kw)) + OV(m) != 0)
-                    za_ = lds.za[ly][OH(m) ? 0 : 1] * (s_v[e] - s_v[kw]);
-                if (OU(m) + OU(M(ks)) != 0) {
-                    const T bcH = OH(m) ? T(1) : a.lbc;
-                    zb = dvr(bcH * fm(-lds.cu[ly], s_u[ks], lds.cu[ly + 1] * s_u[e]), a.AdT, a.rAdT);
-                }
-                zeta = za_ - dvr(zb, lds.cH[ly], lds.rcH[ly]);
-            }
-            // computePotVort (src/swm_timestep_module.f90:230-257)
-            const T pD = Dh > a.eps ? Dh : a.eps;
-            T Pot;
-            if constexpr (VAR == VAR_MS) {   // (f + zeta_bs) / pD
-                const int gi = wrap(i0 + lx - 1, Nx);
-                Pot = dv(lds.fH[ly] + fldg(a.zbs, (size_t)gj * P + gi, gj, OH(m)), pD);
-                lds.zt[e] = zeta;
-            } else {
-                Pot = FN ? dv(lds.fH[ly] + zeta, pD) : dv(lds.fH[ly], pD);
-            }
-            s_Pot[e] = Pot;
-            // SWM_LateralMixing_compute_p, P_lambda-theta on ocean H points
-            T plt = T(0);
-            if (a.mix && OH(m)) {
-                const T* c = &lds.pltc[ly][(OU(m) * 2 + OU(M(ks))) * 3];
-                plt = Dh * fm(c[2], s_u[ks], fm(c[1], s_u[e], c[0] * (s_v[e] - s_v[kw])));
-            }
-            s_plt[e] = plt;
-            if (interior) { gst(a.diag[1], doff, Dh); gst(a.diag[4], doff, zeta); gst(a.diag[5], doff, Pot); }
+        // computePotVort (src/swm_timestep_module.f90:230-257)
+        const T pD = Dh > a.eps ? Dh : a.eps;
+        T Pot;
+        if constexpr (VAR == VAR_MS) {   // (f + zeta_bs) / pD
+            const int gj = wrap(j0 + ly, Ny), gi = wrap(i0 + lx, Nx);
+            Pot = dv(lds.fH[ly + 1] + fldg(a.zbs, (size_t)gj * P + gi, gj, oh), pD);
+            lds.zt[Q] = zeta;
+        } else {
+            Pot = FN ? dv(lds.fH[ly + 1] + zeta, pD) : dv(lds.fH[ly + 1], pD);
         }
-        // computeD: Du, Dv kept for phase 3 (Du from column 1, Dv from row 1 on)
-        if constexpr (LdsDuDv<T, TX, TY>::SDU)
-            if (lx >= 1) lds.Du[e] = interp_noland2(s_D[e], s_D[e - 1], OE(m), OE(M(e - 1)));
-        if constexpr (LdsDuDv<T, TX, TY>::SDV)
-            if (ly >= 1) lds.Dv[e] = interp_noland2(s_D[e], s_D[e - EW], OE(m), OE(M(e - EW)));
-        if (interior) {   // computeMassFluxes: MU = Du * u on ocean u, MV = Dv * v on ocean v
-            const T Du = interp_noland2(s_D[e], s_D[e - 1], OE(m), OE(M(e - 1)));
-            const T Dv = interp_noland2(s_D[e], s_D[e - EW], OE(m), OE(M(e - EW)));
-            gst(a.diag[2], doff, Du);
-            gst(a.diag[7], doff, OU(m) ? Du * s_u[e] : T(0));
-            gst(a.diag[3], doff, Dv);
-            gst(a.diag[8], doff, OV(m) ? Dv * s_v[e] : T(0));
+        s_Pot[Q] = Pot;
+        // SWM_LateralMixing_compute_p: P_lambda-lambda on ocean eta points,
+        // P_lambda-theta on ocean H points
+        T pll = T(0), plt = T(0);
+        if (opt & OPT_MIX) {
+            const T* const c = &lds.pllc[ly][(((ca >> CC_VN) & 1) * 2 + OV(ca)) * 3];
+            const T p1 = Da * fm(c[2], va, fm(c[1], vc, c[0] * (ub - ua)));
+            pll = oe ? p1 : T(0);
+            const T* const h = &lds.pltc[ly + 1][(OU(cq) * 2 + ((cq >> CC_US) & 1)) * 3];
+            const T p2 = Dh * fm(h[2], ub, fm(h[1], ud, h[0] * (vd - vc)));
+            plt = oh ? p2 : T(0);
         }
-        if (lx <= TX && ly <= TY) {
-            const int ke = e + 1, kn = e + EW;
-            // computeEdens (src/swm_timestep_module.f90:259-310); land keeps 0
-            T Ed = T(0);
-            if (OE(m)) {
-                if (FN) {
-                    const T ue = s_u[ke], uc = s_u[e], vn = s_v[kn], vc = s_v[e];
-                    Ed = fm(a.G, eta_e,
-                            (fm(T(0.5), uc * uc, T(0.5) * (ue * ue)) + fm(T(0.5), vc * vc, T(0.5) * (vn * vn))) / T(2));
-                } else if (VAR == VAR_MS) {   // g*eta + uU + vV
-                    const int gi = wrap(i0 + lx - 1, Nx), gip = gi + 1 == Nx ? 0 : gi + 1;
-                    const int gjp = gj + 1 == Ny ? 0 : gj + 1;
-                    const T ube = fldg(a.ubs, (size_t)gj * P + gip, gj, OU(M(ke)) != 0);
-                    const T ubc = fldg(a.ubs, (size_t)gj * P + gi, gj, OU(m) != 0);
-                    const T vbn = fldg(a.vbs, (size_t)gjp * P + gi, gjp, OV(M(kn)) != 0);
-                    const T vbc = fldg(a.vbs, (size_t)gj * P + gi, gj, OV(m) != 0);
-                    const T ue = s_u[ke], uc = s_u[e], vn = s_v[kn], vc = s_v[e];
-                    Ed = ((T(0.5) * (ue * ube) + T(0.5) * (uc * ubc)) + (T(0.5) * (vn * vbn) + T(0.5) * (vc * vbc))) +
-                         a.G * eta_e;
-                } else {
-                    Ed = a.G * eta_e;
-                }
+        s_pll[A] = pll;
+        s_plt[Q] = plt;
+        // computeD, computeMassFluxes: MU = Du * u on ocean u, MV = Dv * v on ocean v
+        if constexpr (SDU) {
+            const T Du = mid(Db, Da, oe && B(cq, CC_ES)), mu = Du * ub;
+            lds.Du[Es] = Du;
+            lds.MU[Es] = B(cq, CC_US) ? mu : T(0);
+        }
+        if constexpr (SDV) {
+            const T Dv = mid(Dc, Da, oe && B(cq, CC_EW)), mv = Dv * vc;
+            lds.Dv[Nw] = Dv;
+            lds.MV[Nw] = B(cq, CC_VW) ? mv : T(0);
+        }
+        if constexpr (DIAG) {
+            const int iq = i0 + lx, jq = j0 + ly;   // Q's cell
+            if (lx < TX && ly < TY && iq < Nx && jq < Ny) {
+                const size_t o = (size_t)jq * P + iq;
+                gst(a.diag[1], o, Dh); gst(a.diag[4], o, zeta); gst(a.diag[5], o, Pot);
             }
-            s_Ed[e] = Ed;
-            // P_lambda-lambda on ocean eta points
-            T pll = T(0);
-            if (a.mix && OE(m)) {
-                const T* c = &lds.pllc[ly][(OV(M(kn)) * 2 + OV(m)) * 3];
-                pll = s_D[e] * fm(c[2], s_v[e], fm(c[1], s_v[kn], c[0] * (s_u[ke] - s_u[e])));
+            if (lx >= 1 && ly >= 1 && iq - 1 < Nx && jq - 1 < Ny) {   // A's
+                const size_t o = (size_t)(jq - 1) * P + iq - 1;
+                const T Du = mid(Da, s_D[A - 1], oe && B(ca, CC_EW)), Dv = mid(Da, s_D[A - EW], oe && B(ca, CC_ES));
+                gst(a.diag[6], o, oe ? Ed : T(0));
+                gst(a.diag[0], o, FN ? (oe ? Da : T(1)) : fldg(a.He, o, jq - 1, oe));
+                gst(a.diag[2], o, Du);
+                gst(a.diag[3], o, Dv);
+                gst(a.diag[7], o, OU(ca) ? Du * ua : T(0));
+                gst(a.diag[8], o, OV(ca) ? Dv * va : T(0));
             }
-            s_pll[e] = pll;
-            if (interior) { gst(a.diag[6], doff, Ed); gst(a.diag[0], doff, s_D[e]); }
         }
     }
     __syncthreads();
@@ -1017,67 +956,148 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
                 return lds.rt[ly - 1][c ? e0 : e1];
             }
         };
-        // static field at (i, j); e = its rowtab entry, -1 for fields without one
-        auto fl = [&](auto& f, int e, size_t at, bool ocean) -> T {
-            if (f.full) return gld(f.full, at);
-            if (e < 0) return gld(f.rows, 2 * (size_t)j + (ocean ? 0 : 1));
-            return rvs(ocean, e, e + 1);
+        // a static field without a rowtab entry at (i, j)
+        auto fl = [&](auto& f, bool ocean) -> T {
+            return f.full ? gld(f.full, off) : gld(f.rows, 2 * (size_t)j + (ocean ? 0 : 1));
         };
-        // x / (static field at (i, j)); e, er: its rowtab entry and that of its reciprocal
-        auto flq = [&](T x, auto& f, int e, int er, size_t at, bool ocean) -> T {
-            if (f.full) return dv(x, gld(f.full, at));
-            return dvr(x, rvs(ocean, e, e + 1), rvs(ocean, er, er + 1));
+        const int c = M(k), ce = M(ke), cn = M(kn);
+        const bool oh = B(c, 0), ou = B(c, 1), ov = B(c, 2), oe = B(c, 3);
+        const bool oew = B(c, CC_EW), oes = B(c, CC_ES), oesw = B(c, CC_ESW), oee = B(c, CC_EE), oen = B(c, CC_EN);
+        const bool oue = B(c, CC_UE), ovn = B(c, CC_VN);
+        // a static field with a rowtab entry at (i, j): the row's value, or its full array's
+        auto flr = [&](unsigned full, auto& f, bool ocean, int e) -> T {
+            T v = rvs(ocean, e, e + 1);
+            if (opt & full) v = gld(f.full, off);
+            return v;
         };
-        // TRC_coeff magnitude (trc_adv) from the rowtab pair at e
-        auto ta = [&](bool neg, int nummask, int den, int e) -> T {
-            const T v = rvs(den == 1, e, e + 1);
-            if (den == 0) return __builtin_nan("");
-            if (!nummask) return neg ? T(-0.0) : T(0.0);
-            return neg ? -v : v;
+        // integrate_AB (src/time_integration_module.f90:74-112) of one field: x plus
+        // the increments of its history g0, g1 and the new tendency, over the
+        // implicit damping.  FP64 divides by the row's divisor through its
+        // reciprocal; FP32 statics hold 1 - 1/impl, and the increments are added to
+        // the carried pair (x, lo_in).
+        auto ab = [&](T x, T g0, T g1, T g2, unsigned short lo_in, unsigned full, auto& f, bool ocean, int e, int er,
+                      unsigned short& lo) -> T {
+            T b = rvs(ocean, e, e + 1);
+            if constexpr (sizeof(T) == 4) {
+                if (opt & full) b = gld(f.full, off);
+                T inc = d.dtc1 * g0;
+                if (d.tstep >= 2) inc = madd(inc, d.dtc2, g1);
+                if (d.tstep >= 3) inc = madd(inc, d.dtc3, g2);
+                return carry_step(x, lo_in, inc, b, lo);
+            } else {
+                T y = rvs(ocean, er, er + 1);
+                if (opt & full) {
+                    b = gld(f.full, off);
+                    y = T(1) / b;
+                }
+                x = madd(x, d.dtc1, g0);
+                if (d.tstep >= 2) x = madd(x, d.dtc2, g1);
+                if (d.tstep >= 3) x = madd(x, d.dtc3, g2);
+                return dvr(x, b, y);
+            }
         };
-        const uint8_t m = M(k);
-        const int oe = OE(m), ou = OU(m), ov = OV(m), oh = OH(m);
-        constexpr bool SDU = LdsDuDv<T, TX, TY>::SDU, SDV = LdsDuDv<T, TX, TY>::SDV;
-        // Du, Dv at a halo cell: from LDS, or interp2(D, eta2u/eta2v_noland) again
-        auto DUat = [&](int kk) -> T {
-            if constexpr (SDU) return lds.Du[kk];
-            else return interp_noland2(s_D[kk], s_D[kk - 1], OE(M(kk)), OE(M(kk - 1)));
+        // the sections below are scheduled one after another, which keeps each
+        // one's temporaries out of the others' registers
+        constexpr bool SECT = sizeof(T) == 8 && NTRC < 2;
+        auto section = [] {
+            if constexpr (SECT) __builtin_amdgcn_sched_barrier(0);
         };
-        auto DVat = [&](int kk) -> T {
-            if constexpr (SDV) return lds.Dv[kk];
-            else return interp_noland2(s_D[kk], s_D[kk - EW], OE(M(kk)), OE(M(kk - EW)));
-        };
-        const T Du = DUat(k);
-        const T Dv = DVat(k);
-        // computeMassFluxes at the points the stencils need
-        auto MUat = [&](int kk) -> T { return OU(M(kk)) ? DUat(kk) * s_u[kk] : T(0); };
-        auto MVat = [&](int kk) -> T { return OV(M(kk)) ? DVat(kk) * s_v[kk] : T(0); };
-        const T MUk = ou ? Du * s_u[k] : T(0), MVk = ov ? Dv * s_v[k] : T(0);
-        const T MUe = MUat(ke), MUs = MUat(ks), MUse = MUat(kse);
-        const T MVn = MVat(kn), MVw = MVat(kw), MVnw = MVat(knw);
-
+        // Du, Dv at the cell
+        T Du, Dv;
+        if constexpr (SDU) Du = lds.Du[k];
+        else Du = mid(s_D[k], s_D[kw], oe && oew);
+        if constexpr (SDV) Dv = lds.Dv[k];
+        else Dv = mid(s_D[k], s_D[ks], oe && oes);
         // SWM_forcing_update (src/swm_forcing_module.f90:135-170)
-        T Fe = fl(a.Fec, RT_FEC, off, oe);
-        if (a.has_oe) Fe = Fe + (T(2) * (fl(a.oRe, -1, off, oe) * d.oc[2] - fl(a.oIe, -1, off, oe) * d.os[2])) * T(oe);
-        T Fx = fl(a.Fxc, RT_FXC, off, ou);
-        if (a.has_taux && ou) {
-            const T tx = fl(a.taux, RT_TAUX, off, true);
-            Fx = Fx + dv(a.has_tau_scale ? a.tau_scale * tx : tx, a.RHO0 * Du);
+        T Fe = flr(FULL_FEC, a.Fec, oe, RT_FEC), Fx = flr(FULL_FXC, a.Fxc, ou, RT_FXC),
+          Fy = flr(FULL_FYC, a.Fyc, ov, RT_FYC);
+        if (opt & OPT_TAUX) {
+            const T tx = flr(FULL_TAUX, a.taux, true, RT_TAUX);
+            const T f = Fx + dv((opt & OPT_TAUSC) ? a.tau_scale * tx : tx, a.RHO0 * Du);
+            Fx = ou ? f : Fx;
         }
-        if (a.has_ox) Fx = Fx + (T(2) * (fl(a.oRx, -1, off, ou) * d.oc[0] - fl(a.oIx, -1, off, ou) * d.os[0])) * T(ou);
-        T Fy = fl(a.Fyc, RT_FYC, off, ov);
-        if (a.has_tauy && ov) {
-            const T ty = fl(a.tauy, RT_TAUY, off, true);
-            Fy = Fy + dv(a.has_tau_scale ? a.tau_scale * ty : ty, a.RHO0 * Dv);
+        if (opt & OPT_TAUY) {
+            const T ty = flr(FULL_TAUY, a.tauy, true, RT_TAUY);
+            const T f = Fy + dv((opt & OPT_TAUSC) ? a.tau_scale * ty : ty, a.RHO0 * Dv);
+            Fy = ov ? f : Fy;
         }
-        if (a.has_oy) Fy = Fy + (T(2) * (fl(a.oRy, -1, off, ov) * d.oc[1] - fl(a.oIy, -1, off, ov) * d.os[1])) * T(ov);
-        if (a.nstream) apply_streams<T>(a, d, off, ou, ov, oe, Du, Dv, Fx, Fy, Fe);
+        if (opt & (OPT_OX | OPT_OY | OPT_OE | OPT_STREAM)) {
+            if (opt & OPT_OE) Fe = Fe + (T(2) * (fl(a.oRe, oe) * d.oc[2] - fl(a.oIe, oe) * d.os[2])) * T(oe);
+            if (opt & OPT_OX) Fx = Fx + (T(2) * (fl(a.oRx, ou) * d.oc[0] - fl(a.oIx, ou) * d.os[0])) * T(ou);
+            if (opt & OPT_OY) Fy = Fy + (T(2) * (fl(a.oRy, ov) * d.oc[1] - fl(a.oIy, ov) * d.os[1])) * T(ov);
+            if (opt & OPT_STREAM) apply_streams<T>(a, d, off, ou, ov, oe, Du, Dv, Fx, Fy, Fe);
+        }
 
         // SWM_timestep_nonlinear (src/swm_timestep_module.f90:349-443)
-        T Ge = T(0), Gu = T(0), Gv = T(0), Lu = T(0), Lv = T(0);
         // neighbours' offsets for the basic-state terms (LINEARISED_MEAN_STATE)
         const int ipx = i + 1 == Nx ? 0 : i + 1, imx = i == 0 ? Nx - 1 : i - 1, jmx = j == 0 ? Ny - 1 : j - 1;
-        if (oe) {
+        T Lu = T(0), Lv = T(0);
+        section();
+        // mass fluxes MV = Dv * v on ocean v at the points of G_u's stencil
+        T MVk, MVn;
+        {
+            T MVw, MVnw;
+            if constexpr (SDV) {
+                MVk = lds.MV[k]; MVn = lds.MV[kn]; MVw = lds.MV[kw]; MVnw = lds.MV[knw];
+            } else {
+                const T Dw = s_D[kw];
+                const T mk = Dv * s_v[k], mn = mid(s_D[kn], s_D[k], oen && oe) * s_v[kn],
+                        mw = mid(Dw, s_D[kw - EW], oew && oesw) * s_v[kw],
+                        mnw = mid(s_D[knw], Dw, B(cn, CC_EW) && oew) * s_v[knw];
+                MVk = ov ? mk : T(0);
+                MVn = ovn ? mn : T(0);
+                MVw = B(c, CC_VW) ? mw : T(0);
+                MVnw = B(cn, CC_VW) ? mnw : T(0);
+            }
+            const T P2 = fm(T(0.5), s_Pot[k], T(0.5) * s_Pot[kn]);
+            const T M4 = fm(T(0.25), MVk, fm(T(0.25), MVnw, fm(T(0.25), MVw, T(0.25) * MVn)));
+            T g = P2 * M4;
+            if constexpr (VAR == VAR_MS) {   // + interp2(zeta, H2u) * interp4(v_bs, v2u)
+                const T Z2 = T(0.5) * lds.zt[kn] + T(0.5) * lds.zt[k];
+                const T vbn = fldg(a.vbs, (size_t)jp * P + i, jp, ovn);
+                const T vbw = fldg(a.vbs, (size_t)j * P + imx, j, B(c, CC_VW));
+                const T vbnw = fldg(a.vbs, (size_t)jp * P + imx, jp, B(cn, CC_VW));
+                const T vbk = fldg(a.vbs, off, j, ov);
+                g = g + Z2 * (((T(0.25) * vbn + T(0.25) * vbw) + T(0.25) * vbnw) + T(0.25) * vbk);
+            }
+            g = g - dvr(s_Ed[k] - s_Ed[kw], rv(RT_EDU, 0), rv(RT_REDU, 0));
+            if (opt & OPT_QUAD) {
+                const T vi = ((T(0.25) * s_v[kn] + T(0.25) * s_v[kw]) + T(0.25) * s_v[knw]) + T(0.25) * s_v[k];
+                const T uc = s_u[k];
+                T qf = fl(a.gsu, true) * sqrt(uc * uc + (vi * vi)) * uc;
+                if (opt & OPT_BARO) qf = dv(qf, fl(a.Hu, true));
+                g = g - qf;
+            }
+            if (opt & OPT_MIX) {
+                const bool one = !(oh && B(c, CC_HN));   // o_tmp = max(1, oH + oH(j+1)) is 1
+                const T c0 = rvs(one, RT_LMU, RT_LMU + 3), c1 = rvs(one, RT_LMU + 1, RT_LMU + 4),
+                        c2 = rvs(one, RT_LMU + 2, RT_LMU + 5);
+                Lu = dv(fm(c2, s_plt[k], fm(c1, s_plt[kn], c0 * (s_pll[k] - s_pll[kw]))), Du);
+                Lu = ou ? Lu : T(0);
+                g = g + Lu;
+            }
+            if constexpr (!DIAG) {
+                const T Gu = g + Fx;
+                const T Gu3 = ou ? Gu : pg[q][1];
+                unsigned short lu = 0;
+                const T un = ab(s_u[k], pg[q][0], pg[q][1], Gu3, plo[q][0], FULL_IMU, a.imu, ou, RT_IMU, RT_RIMU, lu);
+                gst(st, (PL_U + 1 - d.cur) * pl + off, un);
+                gst(st, (PL_GU + r2) * pl + off, Gu3);
+                if constexpr (sizeof(T) == 4)
+                    if (opt & OPT_CARRY) gst((unsigned short*)lo_plane(st, pl, PL_LO), off, lu);
+            }
+        }
+        section();
+        // mass fluxes MU = Du * u on ocean u
+        T MUk, MUe;
+        if constexpr (SDU) {
+            MUk = lds.MU[k]; MUe = lds.MU[ke];
+        } else {
+            const T mk = Du * s_u[k], me = mid(s_D[ke], s_D[k], oee && oe) * s_u[ke];
+            MUk = ou ? mk : T(0);
+            MUe = oue ? me : T(0);
+        }
+        {
             const T t1 = dvr(-(MUe - MUk), a.dL, a.rdL);
             const T t2 = dvr(fm(-MVk, rv(RT_CV, 0), MVn * rv(RT_CV, 1)), a.dT, a.rdT);
             T tt = t1 - t2;
@@ -1085,80 +1105,89 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
                 // src/swm_timestep_module.f90:359-365.  The first interpolation is
                 // taken at i index ip1(j) (column j+1 of row j), as the reference
                 // indexes it; rows j < Nx only (create rejects Ny > Nx).
-                const int c = j + 1 == Nx ? 0 : j + 1, cm = c == 0 ? Nx - 1 : c - 1;
+                const int c1 = j + 1 == Nx ? 0 : j + 1, cm = c1 == 0 ? Nx - 1 : c1 - 1;
                 const size_t rc = (size_t)j * P;
-                const T E1 = interp_noland2(gld(se, rc + c), gld(se, rc + cm), OE(gld(a.mask, rc + c)),
+                const T E1 = interp_noland2(gld(se, rc + c1), gld(se, rc + cm), OE(gld(a.mask, rc + c1)),
                                             OE(gld(a.mask, rc + cm)));
-                const T E0 = interp_noland2(lds.et[k], lds.et[kw], oe, OE(M(kw)));
-                const T ube = fldg(a.ubs, (size_t)j * P + ipx, j, OU(M(ke)) != 0);
-                const T ubk = fldg(a.ubs, off, j, ou != 0);
+                const T E0 = interp_noland2(lds.et[k], lds.et[kw], oe, oew);
+                const T ube = fldg(a.ubs, (size_t)j * P + ipx, j, oue);
+                const T ubk = fldg(a.ubs, off, j, ou);
                 tt = tt - dvr(E1 * ube - E0 * ubk, a.dL, a.rdL);
-                const T E2 = interp_noland2(lds.et[kn], lds.et[k], OE(M(kn)), oe);
-                const T E3 = interp_noland2(lds.et[k], lds.et[ks], oe, OE(M(ks)));
-                const T vbn = fldg(a.vbs, (size_t)jp * P + i, jp, OV(M(kn)) != 0);
-                const T vbk = fldg(a.vbs, off, j, ov != 0);
+                const T E2 = interp_noland2(lds.et[kn], lds.et[k], oen, oe);
+                const T E3 = interp_noland2(lds.et[k], lds.et[ks], oe, oes);
+                const T vbn = fldg(a.vbs, (size_t)jp * P + i, jp, ovn);
+                const T vbk = fldg(a.vbs, off, j, ov);
                 tt = tt - dvr((rv(RT_CV, 1) * E2) * vbn - (rv(RT_CV, 0) * E3) * vbk, a.dT, a.rdT);
             }
-            Ge = dvr(tt, rv(RT_ACE, 0), rv(RT_RACE, 0)) + Fe;
+            // land keeps the previous newest tendency, which the reference never
+            // overwrites there
+            const T Ge = dvr(tt, rv(RT_ACE, 0), rv(RT_RACE, 0)) + Fe;
+            if constexpr (!DIAG) {
+                const T Ge3 = oe ? Ge : pg[q][5];
+                unsigned short le = 0;
+                T en = ab(pe[q], pg[q][4], pg[q][5], Ge3, plo[q][2], FULL_IME, a.ime, oe, RT_IME, RT_RIME, le);
+                if (FN) {   // SWM_timestep_step: where (eta < minD - H) eta = minD - H
+                    const T lim = a.minD - flr(FULL_HE, a.He, oe, RT_HE);
+                    le = en < lim ? (unsigned short)0 : le;
+                    en = en < lim ? lim : en;
+                }
+                gst(st, (PL_E + 1 - d.cur) * pl + off, en);
+                gst(st, (PL_GE + r2) * pl + off, Ge3);
+                if constexpr (sizeof(T) == 4)
+                    if (opt & OPT_CARRY) gst((unsigned short*)lo_plane(st, pl, PL_LO + 2), off, le);
+            }
         }
-        if (ou) {
-            const T P2 = fm(T(0.5), s_Pot[k], T(0.5) * s_Pot[kn]);
-            const T M4 = fm(T(0.25), MVk, fm(T(0.25), MVnw, fm(T(0.25), MVw, T(0.25) * MVn)));
-            T g = P2 * M4;
-            if constexpr (VAR == VAR_MS) {   // + interp2(zeta, H2u) * interp4(v_bs, v2u)
-                const T Z2 = T(0.5) * lds.zt[kn] + T(0.5) * lds.zt[k];
-                const T vbn = fldg(a.vbs, (size_t)jp * P + i, jp, OV(M(kn)) != 0);
-                const T vbw = fldg(a.vbs, (size_t)j * P + imx, j, OV(M(kw)) != 0);
-                const T vbnw = fldg(a.vbs, (size_t)jp * P + imx, jp, OV(M(knw)) != 0);
-                const T vbk = fldg(a.vbs, off, j, ov != 0);
-                g = g + Z2 * (((T(0.25) * vbn + T(0.25) * vbw) + T(0.25) * vbnw) + T(0.25) * vbk);
+        section();
+        {
+            T MUs, MUse;
+            if constexpr (SDU) {
+                MUs = lds.MU[ks]; MUse = lds.MU[kse];
+            } else {
+                const T Ds = s_D[ks];
+                const T ms = mid(Ds, s_D[ks - 1], oes && oesw) * s_u[ks],
+                        mse = mid(s_D[kse], Ds, B(ce, CC_ES) && oes) * s_u[kse];
+                MUs = B(c, CC_US) ? ms : T(0);
+                MUse = B(ce, CC_US) ? mse : T(0);
             }
-            g = g - dvr(s_Ed[k] - s_Ed[kw], rv(RT_EDU, 0), rv(RT_REDU, 0));
-            if (a.quad) {
-                const T vi = ((T(0.25) * s_v[kn] + T(0.25) * s_v[kw]) + T(0.25) * s_v[knw]) + T(0.25) * s_v[k];
-                const T uc = s_u[k];
-                T qf = fl(a.gsu, -1, off, true) * sqrt(uc * uc + (vi * vi)) * uc;
-                if (a.barotropic) qf = dv(qf, fl(a.Hu, -1, off, true));
-                g = g - qf;
-            }
-            if (a.mix) {
-                const int ot = (oh + OH(M(kn))) < 1 ? 1 : (oh + OH(M(kn)));
-                const T c0 = rvs(ot == 1, RT_LMU, RT_LMU + 3), c1 = rvs(ot == 1, RT_LMU + 1, RT_LMU + 4),
-                        c2 = rvs(ot == 1, RT_LMU + 2, RT_LMU + 5);
-                Lu = dv(fm(c2, s_plt[k], fm(c1, s_plt[kn], c0 * (s_pll[k] - s_pll[kw]))), Du);
-                g = g + Lu;
-            }
-            Gu = g + Fx;
-        }
-        if (ov) {
             const T P2 = fm(T(0.5), s_Pot[k], T(0.5) * s_Pot[ke]);
             const T M4 = fm(T(0.25), MUse, fm(T(0.25), MUk, fm(T(0.25), MUs, T(0.25) * MUe)));
             T g = -(P2 * M4);
             if constexpr (VAR == VAR_MS) {   // - interp2(zeta, H2v) * interp4(u_bs, u2v)
                 const T Z2 = T(0.5) * lds.zt[ke] + T(0.5) * lds.zt[k];
-                const T ube = fldg(a.ubs, (size_t)j * P + ipx, j, OU(M(ke)) != 0);
-                const T ubs_ = fldg(a.ubs, (size_t)jmx * P + i, jmx, OU(M(ks)) != 0);
-                const T ubk = fldg(a.ubs, off, j, ou != 0);
-                const T ubse = fldg(a.ubs, (size_t)jmx * P + ipx, jmx, OU(M(kse)) != 0);
+                const T ube = fldg(a.ubs, (size_t)j * P + ipx, j, oue);
+                const T ubs_ = fldg(a.ubs, (size_t)jmx * P + i, jmx, B(c, CC_US));
+                const T ubk = fldg(a.ubs, off, j, ou);
+                const T ubse = fldg(a.ubs, (size_t)jmx * P + ipx, jmx, B(ce, CC_US));
                 g = g - Z2 * (((T(0.25) * ube + T(0.25) * ubs_) + T(0.25) * ubk) + T(0.25) * ubse);
             }
             g = g - dvr(s_Ed[k] - s_Ed[ks], a.AdT, a.rAdT);
-            if (a.quad) {
+            if (opt & OPT_QUAD) {
                 const T ui = ((T(0.25) * s_u[ke] + T(0.25) * s_u[ks]) + T(0.25) * s_u[k]) + T(0.25) * s_u[kse];
                 const T vc = s_v[k];
-                T qf = fl(a.gsv, -1, off, true) * sqrt(vc * vc + (ui * ui)) * vc;
-                if (a.barotropic) qf = dv(qf, fl(a.Hv, -1, off, true));
+                T qf = fl(a.gsv, true) * sqrt(vc * vc + (ui * ui)) * vc;
+                if (opt & OPT_BARO) qf = dv(qf, fl(a.Hv, true));
                 g = g - qf;
             }
-            if (a.mix) {
-                const int ot = (oe + OE(M(ks))) < 1 ? 1 : (oe + OE(M(ks)));
-                const T c0 = rvs(ot == 1, RT_LMV, RT_LMV + 3), c1 = rvs(ot == 1, RT_LMV + 1, RT_LMV + 4),
-                        c2 = rvs(ot == 1, RT_LMV + 2, RT_LMV + 5);
+            if (opt & OPT_MIX) {
+                const bool one = !(oe && oes);   // o_tmp = max(1, oeta + oeta(j-1)) is 1
+                const T c0 = rvs(one, RT_LMV, RT_LMV + 3), c1 = rvs(one, RT_LMV + 1, RT_LMV + 4),
+                        c2 = rvs(one, RT_LMV + 2, RT_LMV + 5);
                 Lv = dv(fm(c2, s_pll[ks], fm(c1, s_pll[k], c0 * (s_plt[ke] - s_plt[k]))), Dv);
+                Lv = ov ? Lv : T(0);
                 g = g + Lv;
             }
-            Gv = g + Fy;
+            if constexpr (!DIAG) {
+                const T Gv = g + Fy;
+                const T Gv3 = ov ? Gv : pg[q][3];
+                unsigned short lv = 0;
+                const T vn = ab(s_v[k], pg[q][2], pg[q][3], Gv3, plo[q][1], FULL_IMV, a.imv, ov, RT_IMV, RT_RIMV, lv);
+                gst(st, (PL_V + 1 - d.cur) * pl + off, vn);
+                gst(st, (PL_GV + r2) * pl + off, Gv3);
+                if constexpr (sizeof(T) == 4)
+                    if (opt & OPT_CARRY) gst((unsigned short*)lo_plane(st, pl, PL_LO + 1), off, lv);
+            }
         }
+        section();
 
         if (DIAG) {
             gst(a.diag[9], off, Fx); gst(a.diag[10], off, Fy); gst(a.diag[11], off, Fe);
@@ -1173,135 +1202,91 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
             continue;
         }
 
-        // integrate_AB (src/time_integration_module.f90:74-112); land keeps the
-        // previous newest tendency, which the reference never overwrites there.
-        const T Gu3 = ou ? Gu : pg[q][1];
-        const T Gv3 = ov ? Gv : pg[q][3];
-        const T Ge3 = oe ? Ge : pg[q][5];
-        // the damping static at (i, j): FP32 contexts hold 1 - 1/impl there
-        auto fdv = [&](auto& f, int e, bool ocean) -> T { return f.full ? gld(f.full, off) : rvs(ocean, e, e + 1); };
-        T un, vn, en;
-        unsigned short lu = 0, lv = 0, le = 0;
-        if constexpr (sizeof(T) == 4) {   // increments added to the carried pair
-            T iu = d.dtc1 * pg[q][0], iv = d.dtc1 * pg[q][2], ie = d.dtc1 * pg[q][4];
-            if (d.tstep >= 2) {
-                iu = madd(iu, d.dtc2, pg[q][1]);
-                iv = madd(iv, d.dtc2, pg[q][3]);
-                ie = madd(ie, d.dtc2, pg[q][5]);
-            }
-            if (d.tstep >= 3) {
-                iu = madd(iu, d.dtc3, Gu3);
-                iv = madd(iv, d.dtc3, Gv3);
-                ie = madd(ie, d.dtc3, Ge3);
-            }
-            un = carry_step(s_u[k], plo[q][0], iu, fdv(a.imu, RT_IMU, ou), lu);
-            vn = carry_step(s_v[k], plo[q][1], iv, fdv(a.imv, RT_IMV, ov), lv);
-            en = carry_step(pe[q], plo[q][2], ie, fdv(a.ime, RT_IME, oe), le);
-        } else {
-            un = s_u[k], vn = s_v[k], en = pe[q];
-            un = madd(un, d.dtc1, pg[q][0]);
-            vn = madd(vn, d.dtc1, pg[q][2]);
-            en = madd(en, d.dtc1, pg[q][4]);
-            if (d.tstep >= 2) {
-                un = madd(un, d.dtc2, pg[q][1]);
-                vn = madd(vn, d.dtc2, pg[q][3]);
-                en = madd(en, d.dtc2, pg[q][5]);
-            }
-            if (d.tstep >= 3) {
-                un = madd(un, d.dtc3, Gu3);
-                vn = madd(vn, d.dtc3, Gv3);
-                en = madd(en, d.dtc3, Ge3);
-            }
-            un = flq(un, a.imu, RT_IMU, RT_RIMU, off, ou);
-            vn = flq(vn, a.imv, RT_IMV, RT_RIMV, off, ov);
-            en = flq(en, a.ime, RT_IME, RT_RIME, off, oe);
-        }
-        if (FN) {   // SWM_timestep_step: where (eta < minD - H) eta = minD - H
-            const T lim = a.minD - fl(a.He, RT_HE, off, oe);
-            if (en < lim) { en = lim; le = 0; }
-        }
-        gst(st, (PL_U + 1 - d.cur) * pl + off, un);
-        gst(st, (PL_V + 1 - d.cur) * pl + off, vn);
-        gst(st, (PL_E + 1 - d.cur) * pl + off, en);
-        if constexpr (sizeof(T) == 4) {
-            if (a.carry) {
-                gst((unsigned short*)lo_plane(st, pl, PL_LO), off, lu);
-                gst((unsigned short*)lo_plane(st, pl, PL_LO + 1), off, lv);
-                gst((unsigned short*)lo_plane(st, pl, PL_LO + 2), off, le);
-            }
-        }
-        gst(st, (PL_GU + r2) * pl + off, Gu3);
-        gst(st, (PL_GV + r2) * pl + off, Gv3);
-        gst(st, (PL_GE + r2) * pl + off, Ge3);
-
         // TRC_tracer_incr + TRC_tracer_integrate (src/tracer_module.f90:154-232)
 #pragma unroll
         for (int n = 0; n < NTRC; ++n) {
             T* const tb = st + (PL_TRC + PL_PER_TRC * n) * pl;
-            const T CH = s_CH[n][k], CHe = s_CH[n][ke], CHw = s_CH[n][kw], CHn = s_CH[n][kn], CHs = s_CH[n][ks];
-            const T C = s_C[n][k], Ce = s_C[n][ke], Cw = s_C[n][kw], Cn = s_C[n][kn], Cs = s_C[n][ks];
-            // tracer velocities are the master fields (model_advance,
-            // src/model.f90:238-259): u = 0, += ocean_u * DYNFROMFILE data
-            // (DFF_advance, src/dynFromFile_module.f90:137-160), += SWM_u
-            T um = T(0) + s_u[k], ume = T(0) + s_u[ke], vm = T(0) + s_v[k], vmn = T(0) + s_v[kn];
-            const uint8_t me = M(ke), mw = M(kw), mn = M(kn), ms = M(ks);
-            if (DYN && a.dyn_u) {
-                const size_t offe = (size_t)j * P + (i + 1 == Nx ? 0 : i + 1);
-                um = (T(0) + T(ou) * dyn_val(a.dyn_u, d.ds[0], off)) + s_u[k];
-                ume = (T(0) + T(OU(me)) * dyn_val(a.dyn_u, d.ds[0], offe)) + s_u[ke];
-            }
-            if (DYN && a.dyn_v) {
-                const size_t offn = (size_t)jp * P + i;
-                vm = (T(0) + T(ov) * dyn_val(a.dyn_v, d.ds[1], off)) + s_v[k];
-                vmn = (T(0) + T(OV(mn)) * dyn_val(a.dyn_v, d.ds[1], offn)) + s_v[kn];
-            }
-            const int oee = OE(me), oew = OE(mw), oen = OE(mn), oes = OE(ms);
-            const int oue = OU(me), ovn = OV(mn);
-            T diff = T(0);
-            if (oe) {
+            const int rt = RT_TRC + RT_PER_TRC * n;
+            const unsigned full = FULL_TRC << (3 * n);   // timpl, gC, C0
+            // the cell's index anew: what this section reads of D and the codes
+            // is read again rather than held through the momentum sections
+            int kt = k;
+            if constexpr (SECT) asm volatile("" : "+v"(kt));
+            const int c = M(kt);
+            const bool ou = B(c, 1), ov = B(c, 2), oe = B(c, 3);
+            const bool oew = B(c, CC_EW), oes = B(c, CC_ES), oee = B(c, CC_EE), oen = B(c, CC_EN);
+            const bool oue = B(c, CC_UE), ovn = B(c, CC_VN);
+            const T C = s_C[n][kt];
+            T g;   // diffusion
+            {
+                T Du, Dv, hue, hvn;   // hue, hvn: Du(i+1,j), Dv(i,j+1)
+                if constexpr (SDU) {
+                    Du = lds.Du[kt]; hue = lds.Du[kt + 1];
+                    Dv = lds.Dv[kt]; hvn = lds.Dv[kt + EW];
+                } else {
+                    const T Dk = s_D[kt];
+                    Du = mid(Dk, s_D[kt - 1], oe && oew);
+                    hue = mid(s_D[kt + 1], Dk, oee && oe);
+                    Dv = mid(Dk, s_D[kt - EW], oe && oes);
+                    hvn = mid(s_D[kt + EW], Dk, oen && oe);
+                }
                 const T kap = a.kappa[n];
-                const T hue = DUat(ke);   // interp2 of D(i+1,j), D(i,j)
-                const T hvn = DVat(kn);   // interp2 of D(i,j+1), D(i,j)
-                const T c9 = oue ? rv(RT_T9, 0) : T(0.0);
-                const T c10 = ou ? -rv(RT_T9, 0) : T(-0.0);
-                const T c11 = ovn ? rv(RT_T11, 0) : T(0.0);
-                const T c12 = ov ? -rv(RT_T12, 0) : T(-0.0);
-                diff = fm((kap * Dv) * (C - Cs), c12,
-                          fm((kap * hvn) * (Cn - C), c11, fm((kap * Du) * (C - Cw), c10, ((kap * hue) * (Ce - C)) * c9)));
+                const T t9 = rv(RT_T9, 0), t11 = rv(RT_T11, 0), t12 = rv(RT_T12, 0);
+                const T c9 = oue ? t9 : T(0.0);
+                const T c10 = ou ? -t9 : T(-0.0);
+                const T c11 = ovn ? t11 : T(0.0);
+                const T c12 = ov ? -t12 : T(-0.0);
+                const T diff =
+                    fm((kap * Dv) * (C - s_C[n][kt - EW]), c12,
+                       fm((kap * hvn) * (s_C[n][kt + EW] - C), c11,
+                          fm((kap * Du) * (C - s_C[n][kt - 1]), c10, ((kap * hue) * (s_C[n][kt + 1] - C)) * c9)));
+                g = oe ? diff : T(0);
             }
-            const T c1 = ta(true, oue & oee, oee + oe, RT_TA);
-            const T c2 = ta(false, ou & oew, oew + oe, RT_TA);
-            const T c3 = ta(true, ovn & oen, oen + oe, RT_TB);
-            const T c4 = ta(false, ov & oes, oes + oe, RT_TC);
-            const T c5 = ta(true, oue & oe, oee + oe, RT_TA);
-            const T c6 = ta(false, ou & oe, oew + oe, RT_TA);
-            const T c7 = ta(true, ovn & oe, oen + oe, RT_TB);
-            const T c8 = ta(false, ov & oe, oes + oe, RT_TC);
-            T g = fm(CHw * um, c2, (CHe * ume) * c1);
-            g = fm(CHn * vmn, c3, g);
-            g = fm(CHs * vm, c4, g);
-            g = fm(CH * ume, c5, g);
-            g = fm(CH * um, c6, g);
-            g = fm(CH * vmn, c7, g);
-            g = fm(CH * vm, c8, g);
-            g = g + diff;
-            g = fm(-(fl(a.gC[n], RT_TRC + RT_PER_TRC * n + 2, off, oe) * s_D[k]),
-                   C - fl(a.C0[n], RT_TRC + RT_PER_TRC * n + 4, off, oe), g);
+            section();
+            const T CH = s_CH[n][kt];
+            {
+                // tracer velocities are the master fields (model_advance,
+                // src/model.f90:238-259): u = 0, += ocean_u * DYNFROMFILE data
+                // (DFF_advance, src/dynFromFile_module.f90:137-160), += SWM_u
+                T um = T(0) + s_u[kt], ume = T(0) + s_u[kt + 1], vm = T(0) + s_v[kt], vmn = T(0) + s_v[kt + EW];
+                if (DYN && (opt & OPT_DYN)) {
+                    if (a.dyn_u) {
+                        um = (T(0) + T(ou) * dyn_val(a.dyn_u, d.ds[0], off)) + s_u[kt];
+                        ume = (T(0) + T(oue) * dyn_val(a.dyn_u, d.ds[0], (size_t)j * P + ipx)) + s_u[kt + 1];
+                    }
+                    if (a.dyn_v) {
+                        vm = (T(0) + T(ov) * dyn_val(a.dyn_v, d.ds[1], off)) + s_v[kt];
+                        vmn = (T(0) + T(ovn) * dyn_val(a.dyn_v, d.ds[1], (size_t)jp * P + i)) + s_v[kt + EW];
+                    }
+                }
+                // TRC_coeff magnitude (trc_adv) of a face: 0/0 (NaN) between two land cells
+                auto face = [&](bool nb, int e) -> T {
+                    const T v = rvs(nb != oe, e, e + 1);
+                    return nb || oe ? v : T(__builtin_nan(""));
+                };
+                // signed coefficient: zero (with the sign) where the mask product is 0
+                auto sg = [&](bool neg, bool on, T v) -> T {
+                    const T x = on || !(v == v) ? v : T(0.0);
+                    return neg ? -x : x;
+                };
+                const T fe = face(oee, RT_TA), fw = face(oew, RT_TA), fn = face(oen, RT_TB), fs = face(oes, RT_TC);
+                T f = fm(s_CH[n][kt - 1] * um, sg(false, ou && oew, fw),
+                         (s_CH[n][kt + 1] * ume) * sg(true, oue && oee, fe));
+                f = fm(s_CH[n][kt + EW] * vmn, sg(true, ovn && oen, fn), f);
+                f = fm(s_CH[n][kt - EW] * vm, sg(false, ov && oes, fs), f);
+                f = fm(CH * ume, sg(true, oue && oe, fe), f);
+                f = fm(CH * um, sg(false, ou && oe, fw), f);
+                f = fm(CH * vmn, sg(true, ovn && oe, fn), f);
+                f = fm(CH * vm, sg(false, ov && oe, fs), f);
+                g = f + g;
+            }
+            const T gC = flr(full << 1, a.gC[n], oe, rt + 2), C0 = flr(full << 2, a.C0[n], oe, rt + 4);
+            g = fm(-(gC * (oe ? s_D[kt] : T(1))), C - C0, g);   // D = 1 on land (tracers are FULLY_NONLINEAR)
             g = fm(C, Fe, g);   // + C * Fe
-            T chn;
-            if constexpr (sizeof(T) == 4) {
-                T inc = d.dtc1 * pt[q][n][0];
-                if (d.tstep >= 2) inc = madd(inc, d.dtc2, pt[q][n][1]);
-                if (d.tstep >= 3) inc = madd(inc, d.dtc3, g);
-                unsigned short lc;
-                chn = carry_step(CH, plo[q][3 + n], inc, fdv(a.timpl[n], RT_TRC + RT_PER_TRC * n, oe), lc);
-                if (a.carry) gst((unsigned short*)lo_plane(tb, pl, PL_TLO), off, lc);
-            } else {
-                chn = CH + d.dtc1 * pt[q][n][0];
-                if (d.tstep >= 2) chn = madd(chn, d.dtc2, pt[q][n][1]);
-                if (d.tstep >= 3) chn = madd(chn, d.dtc3, g);
-                chn = flq(chn, a.timpl[n], RT_TRC + RT_PER_TRC * n, RT_TRC + RT_PER_TRC * n + 6, off, oe);
-            }
+            unsigned short lc = 0;
+            const T chn = ab(CH, pt[q][n][0], pt[q][n][1], g, plo[q][3 + n], full, a.timpl[n], oe, rt, rt + 6, lc);
+            if constexpr (sizeof(T) == 4)
+                if (opt & OPT_CARRY) gst((unsigned short*)lo_plane(tb, pl, PL_TLO), off, lc);
             gst(tb, (1 - d.cur) * pl + off, chn);
             gst(tb, (2 + r2) * pl + off, g);
         }
@@ -1316,6 +1301,15 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
 // than the mask arithmetic saves (7 % with every tile on the OCEAN path).
 template <typename T>
 inline constexpr bool kOceanSplit = sizeof(T) == 4;
+
+// The thread's index in its block, for a tile inside a loop over tiles: not
+// known to be the same in every round, so that the tile's LDS addresses are
+// formed where they are used instead of held in registers round the loop.
+__device__ __forceinline__ int loop_tid() {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    return tid;
+}
 
 // One 256-thread block advances tile t (TX x TY cells) of the domain in d by
 // one step.  L is a TileLds with room for at least NTRC tracers.
@@ -1335,24 +1329,24 @@ inline constexpr bool kOceanSplit = sizeof(T) == 4;
 // kernels set it for FP32 (kOceanSplit).
 template <typename T, int VAR, int NTRC, int TX, int TY, bool DIAG, bool LATE = false, bool DYN = true,
           bool OSPLIT = false, typename L>
-__device__ __forceinline__ void tile_body(const Dyn<T>& d, const int t, L& lds) {
+__device__ __forceinline__ void tile_body(const Dyn<T>& d, const int t, L& lds, const int tid) {
     using S = TileShapeC<TX, TY>;
     TileRegs<T, S::NE, S::NO, (NTRC > 0 ? NTRC : 1), RowTabC<TX, TY, NTRC>::NQ> R;
-    tile_load<T, VAR, NTRC, TX, TY, DIAG, !LATE>(d, t, R);
-    tile_stage<T, VAR, NTRC, TX, TY, DIAG>(d, t, R, lds);
-    if (LATE) tile_load_hist<T, VAR, NTRC, TX, TY, DIAG>(d, t, R);
+    tile_load<T, VAR, NTRC, TX, TY, DIAG, !LATE>(d, t, R, tid);
+    tile_stage<T, VAR, NTRC, TX, TY, DIAG>(d, t, R, lds, tid);
+    if (LATE) tile_load_hist<T, VAR, NTRC, TX, TY, DIAG>(d, t, R, tid);
     if constexpr (OSPLIT && !DIAG) {
         static_assert(S::NT == 256, "four wavefronts vote");
         const int w = __all(R.ocean);
-        if ((threadIdx.x & 63) == 0) lds.ocean[threadIdx.x >> 6] = w;
+        if ((tid & 63) == 0) lds.ocean[tid >> 6] = w;
         __syncthreads();
         if (lds.ocean[0] & lds.ocean[1] & lds.ocean[2] & lds.ocean[3])
-            tile_compute<T, VAR, NTRC, TX, TY, DIAG, DYN, true>(d, t, lds, R.g, R.gt, R.eo, R.lo);
+            tile_compute<T, VAR, NTRC, TX, TY, DIAG, DYN, true>(d, t, lds, R.g, R.gt, R.eo, R.lo, tid);
         else
-            tile_compute<T, VAR, NTRC, TX, TY, DIAG, DYN, false>(d, t, lds, R.g, R.gt, R.eo, R.lo);
+            tile_compute<T, VAR, NTRC, TX, TY, DIAG, DYN, false>(d, t, lds, R.g, R.gt, R.eo, R.lo, tid);
     } else {
         __syncthreads();
-        tile_compute<T, VAR, NTRC, TX, TY, DIAG, DYN>(d, t, lds, R.g, R.gt, R.eo, R.lo);
+        tile_compute<T, VAR, NTRC, TX, TY, DIAG, DYN>(d, t, lds, R.g, R.gt, R.eo, R.lo, tid);
     }
 }
 
@@ -1361,9 +1355,9 @@ __global__ void __launch_bounds__(256)
 step_kernel(const Dyn<T> d) {
     using DD = LdsDuDv<T, TX, TY>;
     using RTC = RowTabC<TX, TY, NTRC>;
-    __shared__ TileLds<T, (NTRC > 0 ? NTRC : 1), (TX + 2) * (TY + 2), TY + 2,
+    __shared__ TileLds<T, NTRC, (TX + 2) * (TY + 2), TY + 2,
                        (VAR == VAR_MS ? (TX + 2) * (TY + 2) : 1), DD::DUE, DD::DVE, RTC::LR, RTC::LK> lds;
-    tile_body<T, VAR, NTRC, TX, TY, DIAG, LATE, true, kOceanSplit<T>>(d, xcd_tile(blockIdx.x, d.nblk), lds);
+    tile_body<T, VAR, NTRC, TX, TY, DIAG, LATE, true, kOceanSplit<T>>(d, xcd_tile(blockIdx.x, d.nblk), lds, threadIdx.x);
 }
 
 // Persistent tile kernel: block b advances the tiles [b*tpb, (b+1)*tpb) in
@@ -1377,16 +1371,17 @@ step_kernel_p(const Dyn<T> d) {
     constexpr int NTR = NTRC > 0 ? NTRC : 1;
     using DD = LdsDuDv<T, TX, TY>;
     using RTC = RowTabC<TX, TY, NTRC>;
-    __shared__ TileLds<T, NTR, S::E, S::EH, 1, DD::DUE, DD::DVE, RTC::LR, RTC::LK> lds;
+    __shared__ TileLds<T, NTRC, S::E, S::EH, 1, DD::DUE, DD::DVE, RTC::LR, RTC::LK> lds;
     const int b = xcd_tile(blockIdx.x, gridDim.x);
     const int t0 = b * d.tpb;
     const int t1 = t0 + d.tpb < d.nblk ? t0 + d.tpb : d.nblk;
     if (t0 >= t1) return;   // whole block
     TileRegs<T, S::NE, S::NO, NTR, RTC::NQ> R;
-    tile_load<T, VAR, NTRC, TX, TY, false>(d, t0, R);
+    tile_load<T, VAR, NTRC, TX, TY, false>(d, t0, R, threadIdx.x);
     for (int t = t0; t < t1; ++t) {
+        const int tid = loop_tid();
         if (t > t0) __syncthreads();   // phase 3 of the previous tile is done with LDS
-        tile_stage<T, VAR, NTRC, TX, TY, false>(d, t, R, lds);
+        tile_stage<T, VAR, NTRC, TX, TY, false>(d, t, R, lds, tid);
         T g[S::NO][6], gt[S::NO][NTR][2], eo[S::NO];
         unsigned short lo[S::NO][3 + NTR];
 #pragma unroll
@@ -1400,8 +1395,8 @@ step_kernel_p(const Dyn<T> d) {
             for (int n = 0; n < NTR; ++n) { gt[q][n][0] = R.gt[q][n][0]; gt[q][n][1] = R.gt[q][n][1]; }
         }
         __syncthreads();
-        if (t + 1 < t1) tile_load<T, VAR, NTRC, TX, TY, false>(d, t + 1, R);
-        tile_compute<T, VAR, NTRC, TX, TY, false>(d, t, lds, g, gt, eo, lo);
+        if (t + 1 < t1) tile_load<T, VAR, NTRC, TX, TY, false>(d, t + 1, R, tid);
+        tile_compute<T, VAR, NTRC, TX, TY, false>(d, t, lds, g, gt, eo, lo, tid);
     }
 }
 
@@ -1433,7 +1428,7 @@ struct MemberStep {
 // Work item w of a batched step: tile (w - wbase) of member owner[w].
 template <typename T, int VAR, int NTRC_MAX, int TX, int TY, typename L>
 __device__ __forceinline__ void batch_item(const Member<T>* __restrict__ mem, const MemberStep* __restrict__ stp,
-                                           const int* __restrict__ owner, const int w, L& lds) {
+                                           const int* __restrict__ owner, const int w, L& lds, const int tid) {
     const int lo = owner[w];   // member whose work range holds w
     const Member<T>& m = mem[lo];
     const MemberStep ms = stp[lo];
@@ -1456,14 +1451,14 @@ __device__ __forceinline__ void batch_item(const Member<T>* __restrict__ mem, co
     d.dtc3 = m.dtc[tstep - 1][2];
     const int t = w - m.wbase;
     if constexpr (NTRC_MAX == 0) {
-        tile_body<T, VAR, 0, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds);
+        tile_body<T, VAR, 0, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds, tid);
     } else if constexpr (NTRC_MAX == 1) {
-        if (m.ntr == 0) tile_body<T, VAR, 0, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds);
-        else tile_body<T, VAR, 1, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds);
+        if (m.ntr == 0) tile_body<T, VAR, 0, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds, tid);
+        else tile_body<T, VAR, 1, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds, tid);
     } else {
-        if (m.ntr == 0) tile_body<T, VAR, 0, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds);
-        else if (m.ntr == 1) tile_body<T, VAR, 1, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds);
-        else tile_body<T, VAR, 2, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds);
+        if (m.ntr == 0) tile_body<T, VAR, 0, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds, tid);
+        else if (m.ntr == 1) tile_body<T, VAR, 1, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds, tid);
+        else tile_body<T, VAR, 2, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds, tid);
     }
 }
 
@@ -1511,9 +1506,9 @@ batch_kernel(const Member<T>* __restrict__ mem, const MemberStep* __restrict__ s
              int nwork) {
     using DD = LdsDuDv<T, TX, TY>;
     using RTC = RowTabC<TX, TY, NTRC_MAX>;
-    __shared__ TileLds<T, (NTRC_MAX > 0 ? NTRC_MAX : 1), (TX + 2) * (TY + 2), TY + 2, 1, DD::DUE, DD::DVE, RTC::LR,
+    __shared__ TileLds<T, NTRC_MAX, (TX + 2) * (TY + 2), TY + 2, 1, DD::DUE, DD::DVE, RTC::LR,
                        RTC::LK> lds;
-    batch_item<T, VAR, NTRC_MAX, TX, TY>(mem, stp, owner, xcd_tile(blockIdx.x, nwork), lds);
+    batch_item<T, VAR, NTRC_MAX, TX, TY>(mem, stp, owner, xcd_tile(blockIdx.x, nwork), lds, threadIdx.x);
 }
 
 // model_advance after a batch_kernel step (one thread per member)
@@ -1539,7 +1534,7 @@ batch_queue_kernel(const Member<T>* __restrict__ mem, MemberStep* __restrict__ s
                    const int* __restrict__ owner, int nwork, int nmem, int* __restrict__ queue) {
     using DD = LdsDuDv<T, TX, TY>;
     using RTC = RowTabC<TX, TY, NTRC_MAX>;
-    __shared__ TileLds<T, (NTRC_MAX > 0 ? NTRC_MAX : 1), (TX + 2) * (TY + 2), TY + 2, 1, DD::DUE, DD::DVE, RTC::LR,
+    __shared__ TileLds<T, NTRC_MAX, (TX + 2) * (TY + 2), TY + 2, 1, DD::DUE, DD::DVE, RTC::LR,
                        RTC::LK> lds;
     __shared__ int s_item;
     const int q0 = nwork >> 3, r0 = nwork & 7;
@@ -1563,7 +1558,7 @@ batch_queue_kernel(const Member<T>* __restrict__ mem, MemberStep* __restrict__ s
         const int kend = k + kQueueChunk < n ? k + kQueueChunk : n;
         for (int kk = k; kk < kend; ++kk) {
             if (kk > k) __syncthreads();   // the previous tile is done with LDS
-            batch_item<T, VAR, NTRC_MAX, TX, TY>(mem, stp, owner, lo + kk, lds);
+            batch_item<T, VAR, NTRC_MAX, TX, TY>(mem, stp, owner, lo + kk, lds, loop_tid());
         }
     }
     batch_finish(stp, nmem, queue);
