@@ -1041,13 +1041,21 @@ int step_one(swm_ctx* c) {
     c->ring = (c->ring + 1) % 3;
     for (auto& tr : c->trc) tr.cbuf_valid = false;
     // averaging diag tasks: add dt * field**p of the new N0 (Diag after model_advance)
-    for (auto& av : c->avgs) {
-        const int pl = av.field == 0 ? swm::PL_U + c->cur : av.field == 1 ? swm::PL_V + c->cur
-                     : av.field == 2 ? swm::PL_E + c->cur : swm::PL_TRC + swm::PL_PER_TRC * av.tracer + c->cur;
-        const long n = (long)c->Nx * c->Ny;
-        hipLaunchKernelGGL(swm::avg_accumulate<T>, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->Nx, c->Ny, c->P,
-                           (const T*)plane_ptr(c, pl), av.buf, c->d.dt, av.square);
-        av.weight += c->d.dt;
+    const long pairs = (long)c->P * c->Ny / 2;   // the pitch is even
+    for (size_t k0 = 0; k0 < c->avgs.size(); k0 += swm::kAvgs) {
+        swm::AvgOps<T> ops{};
+        const unsigned n = (unsigned)std::min<size_t>(swm::kAvgs, c->avgs.size() - k0);
+        for (unsigned k = 0; k < n; ++k) {
+            auto& av = c->avgs[k0 + k];
+            const int pl = av.field == 0 ? swm::PL_U + c->cur : av.field == 1 ? swm::PL_V + c->cur
+                         : av.field == 2 ? swm::PL_E + c->cur : swm::PL_TRC + swm::PL_PER_TRC * av.tracer + c->cur;
+            ops.f[k] = (const T*)plane_ptr(c, pl);
+            ops.buf[k] = av.buf;
+            ops.square |= av.square ? 1u << k : 0u;
+            av.weight += c->d.dt;
+        }
+        hipLaunchKernelGGL(swm::avg_accumulate<T>, dim3((unsigned)((pairs + 255) / 256), n), dim3(256), 0, c->stream,
+                           ops, pairs, c->d.dt);
     }
     return 0;
 }
