@@ -1507,14 +1507,12 @@ int psi_t(swm_ctx* c, const double* und = nullptr, const double* vnd = nullptr) 
     const long n = (long)c->Nx * c->Ny;
     hipLaunchKernelGGL(swm::psi_prep<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, sp, u, v, und,
                        vnd, c->psi_buf[0], c->psi_buf[1]);
-    hipLaunchKernelGGL(swm::psi_col<T>, dim3((c->Nx + 255) / 256), dim3(256), 0, c->stream, sp,
-                       (const double*)c->psi_buf[0], c->psi_buf[2], c->psi_buf[3]);
-    const unsigned segs = (unsigned)((c->Nx - 1 + 255) / 256);
-    hipLaunchKernelGGL(swm::psi_row<T>, dim3(segs, 1), dim3(256), 0, c->stream, sp, 0,
-                       (const double*)c->psi_buf[1], (const double*)c->psi_buf[2], c->psi_buf[3]);
-    if (c->Ny > 1)
-        hipLaunchKernelGGL(swm::psi_row<T>, dim3(segs, (unsigned)(c->Ny - 1)), dim3(256), 0, c->stream, sp, 1,
-                           (const double*)c->psi_buf[1], (const double*)c->psi_buf[2], c->psi_buf[3]);
+    hipLaunchKernelGGL(swm::psi_col<T>, dim3((c->Nx + 63) / 64), dim3(64), 0, c->stream, sp,
+                       (const double*)c->psi_buf[0], c->psi_buf[2]);
+    hipLaunchKernelGGL(swm::psi_row<T>, dim3((unsigned)(((c->Nx - 2) / swm::kPsiCells + 1) * c->Ny)), dim3(256), 0,
+                       c->stream, sp, (const double*)c->psi_buf[1], c->psi_buf[3]);
+    hipLaunchKernelGGL(swm::psi_join<T>, dim3((unsigned)(((c->Nx - 1) / 256 + 1) * c->Ny)), dim3(256), 0,
+                       c->stream, sp, (const double*)c->psi_buf[2], c->psi_buf[3]);
     HIPCHK(c, hipGetLastError());
     return 0;
 }

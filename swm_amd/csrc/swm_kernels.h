@@ -2526,58 +2526,132 @@ psi_prep(const Statics<T>* sp, const T* u, const T* v, const double* und, const 
     }
 }
 
-// Column sums sum_{q < j} pu(i, q), one thread per column in order of j; in
-// column Nx they give psi(Nx, j) = -sum * A * dTheta (psi(Nx, 1) = 0).
+// Column sums sum_{q < j} pu(i, q), one thread per column in order of j.  The
+// order leaves one serial chain per column, Nx of them, so the kernel is bound
+// by the latency of its loads: a wavefront per block, to spread the few chains
+// over the CUs, takes kPsiRows rows at once and has the next ones on their way
+// while it adds and stores these.  1024x768: 207 us with blocks of 256 columns,
+// row after row; 17 us.
+constexpr int kPsiRows = 64;
 template <typename T>
-__global__ void __launch_bounds__(256)
-psi_col(const Statics<T>* sp, const double* pu, double* colsum, double* psi) {
-    const Statics<T>& a = *sp;
-    const int Nx = a.Nx, Ny = a.Ny, P = a.P;
-    const int i = blockIdx.x * 256 + threadIdx.x;
+__global__ void __launch_bounds__(64)
+psi_col(const Statics<T>* sp, const double* __restrict__ pu, double* __restrict__ colsum) {
+    const int Nx = sp->Nx, Ny = sp->Ny, P = sp->P;
+    const int i = blockIdx.x * 64 + threadIdx.x;
     if (i >= Nx) return;
-    const double A = (double)a.A, dT = (double)a.dT;
-    double s = 0.0;
-    for (int j = 0; j < Ny; ++j) {
-        const size_t off = (size_t)j * P + i;
-        colsum[off] = s;
-        if (i == Nx - 1) psi[off] = j == 0 ? 0.0 : -s * A * dT;
-        s = s + pu[off];
+    const double* in = pu + i;
+    double* out = colsum + i;
+    double x[kPsiRows], s = 0.0;
+    int j = 0;
+    if (kPsiRows <= Ny) {
+#pragma unroll
+        for (int k = 0; k < kPsiRows; ++k, in += P) x[k] = *in;
+    }
+    for (; j + kPsiRows <= Ny; j += kPsiRows) {
+        double y[kPsiRows] = {};
+        if (j + 2 * kPsiRows <= Ny) {
+#pragma unroll
+            for (int k = 0; k < kPsiRows; ++k, in += P) y[k] = *in;
+        }
+#pragma unroll
+        for (int k = 0; k < kPsiRows; ++k, out += P) {
+            *out = s;
+            s = s + x[k];
+        }
+#pragma unroll
+        for (int k = 0; k < kPsiRows; ++k) x[k] = y[k];
+    }
+#pragma unroll 8
+    for (; j < Ny; ++j, in += P, out += P) {
+        *out = s;
+        s = s + *in;
     }
 }
 
-// Row sums sum_{q = i}^{Nx-1} pv(q, j) for 256 cells of one row per block,
-// each cell adding q = i, i+1, ... in order (rows staged through LDS).  Row 1
-// (j0 = 0) gives psi(i, 1); the interior combines both paths:
-// psi = (-S_row*A*cos_v*dLambda + psi(Nx, j) - S_col*A*dTheta + psi(i, 1)) / 2.
+// Row sums sum_{q = i}^{Nx-2} pv(q, j), each cell adding q = i, i+1, ... in
+// order, times the factors of psi.  That is Nx^2 / 2 additions a row, all cells
+// left of q adding the same pv(q): a wavefront takes 256 cells, four per lane, so
+// that one broadcast of two addends from LDS serves eight additions, the rate at
+// which the four SIMDs of a CU keep LDS and FP64 adders equally busy.
+// A row's left end has the most to add: which wavefront takes which 256 cells
+// turns with the row, so the SIMDs share it.  1024x768: 111 us with one cell per
+// lane, 101 us with that and scalar loads, 33 us so (10 us of additions).
+constexpr int kPsiCells = 1024;   // of one row per block
 template <typename T>
 __global__ void __launch_bounds__(256)
-psi_row(const Statics<T>* sp, int j0, const double* pv, const double* colsum, double* psi) {
+psi_row(const Statics<T>* sp, const double* __restrict__ pv, double* __restrict__ psi) {
+    typedef double pair_t __attribute__((ext_vector_type(2)));
     constexpr int CH = 2048;
-    __shared__ double buf[CH];
+    __shared__ alignas(16) double buf[CH];
     const Statics<T>& a = *sp;
-    const int Nx = a.Nx, P = a.P;
-    const int j = j0 + blockIdx.y;
-    const int i0 = blockIdx.x * 256;
-    const int i = i0 + threadIdx.x;
+    const int Nx = a.Nx, P = a.P, n = Nx - 1;
+    const int nb = (n - 1) / kPsiCells + 1;   // blocks per row
+    const int j = blockIdx.x / nb, lane = threadIdx.x & 63;
+    const int i0 = (blockIdx.x - j * nb) * kPsiCells;
+    const int w = __builtin_amdgcn_readfirstlane(((threadIdx.x >> 6) + j) & 3);
     const double* row = pv + (size_t)j * P;
-    double s = 0.0;
-    for (int c0 = i0; c0 < Nx - 1; c0 += CH) {
-        const int len = min(CH, Nx - 1 - c0);
+    double s[4] = {};
+    for (int c0 = i0; c0 < n; c0 += CH) {
+        const int len = min(CH, n - c0);
         __syncthreads();
         for (int q = threadIdx.x; q < len; q += 256) buf[q] = row[c0 + q];
         __syncthreads();
-        const int qs = max(i - c0, 0);
-        for (int q = qs; q < len; ++q) s = s + buf[q];
+        int q = 0;
+        if (c0 == i0) {   // the wavefront's own cells: cell 64 m + lane starts at its own q
+            q = 256 * w;
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll 4
+                for (int k = 0; k < 64 && q < len; ++k, ++q) {
+                    const double v = buf[q];
+#pragma unroll
+                    for (int c = 0; c < m; ++c) s[c] = s[c] + v;
+                    const double t = s[m] + v;
+                    s[m] = k >= lane ? t : s[m];
+                }
+        }
+        for (; q + 8 <= len; q += 8) {   // q is even here
+            pair_t v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = *(const pair_t*)&buf[q + 2 * k];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) s[c] = s[c] + v[k].x;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) s[c] = s[c] + v[k].y;
+            }
+        }
+        for (; q < len; ++q) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) s[c] = s[c] + buf[q];
+        }
     }
-    if (i >= Nx - 1) return;
-    const double A = (double)a.A, dL = (double)a.dL, dT = (double)a.dT;
-    const double cv = (double)a.cv[j];
-    const size_t off = (size_t)j * P + i;
-    if (j == 0) {
-        psi[off] = -s * A * cv * dL;
-    } else {
-        psi[off] = (-s * A * cv * dL + psi[(size_t)j * P + Nx - 1] - colsum[off] * A * dT + psi[i]) / 2.0;
+    const double A = (double)a.A, dL = (double)a.dL, cv = (double)a.cv[j];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const int i = i0 + 256 * w + 64 * c + lane;
+        if (i < n) psi[(size_t)j * P + i] = -s[c] * A * cv * dL;
     }
+}
+
+// Both paths joined: row 1 of psi_row is psi(i, 1), column Nx gives psi(Nx, j) =
+// -S_col*A*dTheta with psi(Nx, 1) = 0, and in the interior
+// psi = (-S_row*A*cos_v*dLambda + psi(Nx, j) - S_col*A*dTheta + psi(i, 1)) / 2.
+template <typename T>
+__global__ void __launch_bounds__(256)
+psi_join(const Statics<T>* sp, const double* __restrict__ colsum, double* psi) {
+    const Statics<T>& a = *sp;
+    const int n = a.Nx - 1, nb = n / 256 + 1, j = blockIdx.x / nb;
+    const int i = (blockIdx.x - j * nb) * 256 + threadIdx.x;
+    if (i > n) return;
+    const size_t r = (size_t)j * a.P;
+    const double A = (double)a.A, dT = (double)a.dT;
+    const double edge = j == 0 ? 0.0 : -colsum[r + n] * A * dT;
+    if (i == n)
+        psi[r + n] = edge;
+    else if (j > 0)
+        psi[r + i] = (psi[r + i] + edge - colsum[r + i] * A * dT + psi[i]) / 2.0;
 }
 
 template <typename T>
