@@ -248,8 +248,8 @@ struct Dyn {
 
 // A DYNFROMFILE dataset at element off: getChunkData interpolated in time as
 // the forcing streams are (src/memchunk_module.f90:214-243).
-template <typename T>
-__device__ __forceinline__ T dyn_val(const T* r, const SStep<T>& st, size_t off) {
+template <typename T, typename S>
+__device__ __forceinline__ T dyn_val(const T* r, S& st, size_t off) {
     const T y0 = ((const __attribute__((address_space(1))) T*)(r + st.o0))[off];
     if (st.exact) return y0;
     const T y1 = ((const __attribute__((address_space(1))) T*)(r + st.o1))[off];
@@ -381,7 +381,7 @@ struct TileLds {
     static constexpr int RTK = RTK_;
     T u[E], v[E], D[E], Pot[E], Ed[E], pll[E], plt[E];   // D is 0 on land; Ed holds eta until phase 2 replaces it
     T zt[ZE], et[ZE];    // LINEARISED_MEAN_STATE (ZE = E): relative vorticity and eta for phase 3
-    T Du[DUE], Dv[DVE], MU[DUE], MV[DVE];   // interp2(D, eta2u/eta2v_noland) and the mass fluxes (when DUE / DVE = E)
+    T Du[DUE], MU[DUE], MV[DVE];   // interp2(D, eta2u_noland) and the mass fluxes (when DUE / DVE = E)
     T CH[NTR ? NTR : 1][NTR ? E : 1], C[NTR ? NTR : 1][NTR ? E : 1];
     // per-row tables of the EH tile rows (cu also of the row above them)
     T za[EH][2], cu[EH + 1], cH[EH], rcH[EH], fH[EH], pltc[EH][12], pllc[EH][12];
@@ -405,10 +405,12 @@ struct RowTabC {
     static constexpr int NQ = UROW ? 1 : (R * K + 255) / 256;
 };
 
-// Tiles that keep Du, Dv, MU and MV in LDS, computed once per cell in phase 2
+// Tiles that keep Du, MU and MV in LDS, computed once per cell in phase 2
 // instead of at each stencil point in phase 3: the FP32 tiles, which have
-// LDS to spare at their occupancy.  FP64 recomputes them (its tiles would drop
-// to three or four blocks per CU).
+// LDS to spare at their occupancy.  Dv, read at two points, is formed there: with
+// it a 32x8 tile with a tracer takes 21.7 KB and seven blocks fit a CU, without it
+// 20.3 KB and eight do (batched kernel, 14 members: 52.2 -> 50.3 us a step).
+// FP64 recomputes them all (its tiles would drop to three or four blocks per CU).
 template <typename T, int TX, int TY>
 struct LdsDuDv {
     static constexpr int E = (TX + 2) * (TY + 2);
@@ -431,6 +433,21 @@ __device__ __forceinline__ void gst(T* p, size_t i, T v) {
 }
 template <typename T>
 using CStatics = const __attribute__((address_space(4))) Statics<T>;
+// The launch arguments of a kernel whose first argument is a Dyn, for the rare
+// ones among them (the forcing streams' records and phases), read in the branch
+// that uses them.  Named through the Dyn, the compiler reads them on entry and
+// holds them: the step kernels took 106 scalar registers with up to 25 spilled
+// into vector lanes, so FP32 with a tracer had seven of its 16 blocks per CU at
+// 1024^2 resident and two left over.  So they take 56 to 81 and no spills, and
+// FP64 with a tracer 80 vector registers instead of 85: FP32 25.1 -> 22.9 us a
+// step at 1024^2 and 65.9 -> 60.5 at 2304x1800, FP64 38.6 -> 37.5 at 1024^2 and
+// 8.1 -> 7.5 at 96x64.
+template <typename T>
+using CDyn = const __attribute__((address_space(4))) Dyn<T>;
+template <typename T>
+__device__ __forceinline__ CDyn<T>& own_dyn() {
+    return *(CDyn<T>*)__builtin_amdgcn_kernarg_segment_ptr();
+}
 
 // A static field at element offset `at` of row `row` (full array, or the
 // row's ocean / land value), read through the global address space.
@@ -445,8 +462,8 @@ __device__ __forceinline__ auto fldg(const F& f, size_t at, int row, bool ocean)
 // getChunkData (src/memchunk_module.f90:214-243), which interpolates between
 // the bracketing records as interp1D_array2D, y0 + (t-t0)*(y1-y0)/(t1-t0)
 // (src/calc_lib.f90:386-397).  off is the cell's offset within a plane.
-template <typename T, typename S>
-__device__ __forceinline__ void apply_streams(S& a, const Dyn<T>& d, size_t off, int ou, int ov, int oe, T Du, T Dv,
+template <typename T, typename S, typename D>
+__device__ __forceinline__ void apply_streams(S& a, D& d, size_t off, int ou, int ov, int oe, T Du, T Dv,
                                               T& Fx, T& Fy, T& Fe) {
     const int ns = a.nstream;
     // unrolled over the fixed maximum: every d.ss[n] index is a constant, so a
@@ -780,7 +797,7 @@ __device__ __forceinline__ void tile_stage(const Dyn<T>& d, const int t, const R
 // them in the FP64 kernel with a tracer) each waited for its own LDS reads and
 // the phases took 13 000 cycles of a block that had its CU to itself, three
 // times their issue time.
-template <typename T, int VAR, int NTRC, int TX, int TY, bool DIAG, bool DYN = true, bool OCEAN = false, typename L,
+template <typename T, int VAR, int NTRC, int TX, int TY, bool DIAG, bool ALONE = true, bool OCEAN = false, typename L,
           typename G, typename GT, typename GE, typename LO>
 __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& lds, const G& pg, const GT& pt,
                                              const GE& pe, const LO& plo, const int tid) {
@@ -902,8 +919,7 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
             lds.MU[Es] = B(cq, CC_US) ? mu : T(0);
         }
         if constexpr (SDV) {
-            const T Dv = mid(Dc, Da, oe && B(cq, CC_EW)), mv = Dv * vc;
-            lds.Dv[Nw] = Dv;
+            const T mv = mid(Dc, Da, oe && B(cq, CC_EW)) * vc;
             lds.MV[Nw] = B(cq, CC_VW) ? mv : T(0);
         }
         if constexpr (DIAG) {
@@ -1003,11 +1019,9 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
             if constexpr (SECT) __builtin_amdgcn_sched_barrier(0);
         };
         // Du, Dv at the cell
-        T Du, Dv;
+        T Du, Dv = mid(s_D[k], s_D[ks], oe && oes);
         if constexpr (SDU) Du = lds.Du[k];
         else Du = mid(s_D[k], s_D[kw], oe && oew);
-        if constexpr (SDV) Dv = lds.Dv[k];
-        else Dv = mid(s_D[k], s_D[ks], oe && oes);
         // SWM_forcing_update (src/swm_forcing_module.f90:135-170)
         T Fe = flr(FULL_FEC, a.Fec, oe, RT_FEC), Fx = flr(FULL_FXC, a.Fxc, ou, RT_FXC),
           Fy = flr(FULL_FYC, a.Fyc, ov, RT_FYC);
@@ -1021,7 +1035,8 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
             const T f = Fy + dv((opt & OPT_TAUSC) ? a.tau_scale * ty : ty, a.RHO0 * Dv);
             Fy = ov ? f : Fy;
         }
-        if (opt & (OPT_OX | OPT_OY | OPT_OE | OPT_STREAM)) {
+        if (ALONE && (opt & (OPT_OX | OPT_OY | OPT_OE | OPT_STREAM))) {
+            CDyn<T>& d = own_dyn<T>();
             if (opt & OPT_OE) Fe = Fe + (T(2) * (fl(a.oRe, oe) * d.oc[2] - fl(a.oIe, oe) * d.os[2])) * T(oe);
             if (opt & OPT_OX) Fx = Fx + (T(2) * (fl(a.oRx, ou) * d.oc[0] - fl(a.oIx, ou) * d.os[0])) * T(ou);
             if (opt & OPT_OY) Fy = Fy + (T(2) * (fl(a.oRy, ov) * d.oc[1] - fl(a.oIy, ov) * d.os[1])) * T(ov);
@@ -1220,16 +1235,15 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
             T g;   // diffusion
             {
                 T Du, Dv, hue, hvn;   // hue, hvn: Du(i+1,j), Dv(i,j+1)
+                const T Dk = s_D[kt];
                 if constexpr (SDU) {
                     Du = lds.Du[kt]; hue = lds.Du[kt + 1];
-                    Dv = lds.Dv[kt]; hvn = lds.Dv[kt + EW];
                 } else {
-                    const T Dk = s_D[kt];
                     Du = mid(Dk, s_D[kt - 1], oe && oew);
                     hue = mid(s_D[kt + 1], Dk, oee && oe);
-                    Dv = mid(Dk, s_D[kt - EW], oe && oes);
-                    hvn = mid(s_D[kt + EW], Dk, oen && oe);
                 }
+                Dv = mid(Dk, s_D[kt - EW], oe && oes);
+                hvn = mid(s_D[kt + EW], Dk, oen && oe);
                 const T kap = a.kappa[n];
                 const T t9 = rv(RT_T9, 0), t11 = rv(RT_T11, 0), t12 = rv(RT_T12, 0);
                 const T c9 = oue ? t9 : T(0.0);
@@ -1249,7 +1263,8 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
                 // src/model.f90:238-259): u = 0, += ocean_u * DYNFROMFILE data
                 // (DFF_advance, src/dynFromFile_module.f90:137-160), += SWM_u
                 T um = T(0) + s_u[kt], ume = T(0) + s_u[kt + 1], vm = T(0) + s_v[kt], vmn = T(0) + s_v[kt + EW];
-                if (DYN && (opt & OPT_DYN)) {
+                if (ALONE && (opt & OPT_DYN)) {
+                    CDyn<T>& d = own_dyn<T>();
                     if (a.dyn_u) {
                         um = (T(0) + T(ou) * dyn_val(a.dyn_u, d.ds[0], off)) + s_u[kt];
                         ume = (T(0) + T(oue) * dyn_val(a.dyn_u, d.ds[0], (size_t)j * P + ipx)) + s_u[kt + 1];
@@ -1296,9 +1311,9 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
 // Whether the step and batched kernels split off all-ocean tiles (OSPLIT of
 // tile_body): FP32 only.  On the 1024^2 basin with 5 % islands 70 % of the
 // 32x8 tiles are all ocean, and the FP32 step is 6 % faster (31.7 -> 29.8 us).
-// FP64 is 3.7 % slower with it: the two instantiations in one kernel raise its
-// VGPRs from 93 to 107 (four waves per SIMD instead of five), which costs more
-// than the mask arithmetic saves (7 % with every tile on the OCEAN path).
+// FP64 takes 96 VGPRs with both instantiations in one kernel (80 with one) and
+// gains 2 to 4 % from 1024^2 on, but the longer kernel costs 2 to 4 % of the 5 to
+// 8 us of a small grid's step.
 template <typename T>
 inline constexpr bool kOceanSplit = sizeof(T) == 4;
 
@@ -1320,14 +1335,14 @@ __device__ __forceinline__ int loop_tid() {
 // that burst over the barrier and phase 2 (-6 % at 1024^2).  With many rounds
 // the blocks drift apart and the early prefetch hides more latency (+3 % at
 // 2048^2 for the late order).
-// DYN: the tracer may read DYNFROMFILE datasets (contexts that step alone;
-// the batched kernel is built without that branch).
+// ALONE: oscillating and time-interpolated forcing and DYNFROMFILE datasets
+// (contexts that step alone; the batched kernel is built without them).
 // OSPLIT: tiles whose cells and halo are all ocean take tile_compute's
 // OCEAN instantiation.  Each wavefront votes over the masks of its halo cells
 // (already in registers) and writes the vote to LDS before the barrier that
 // follows the stage; no further barrier is needed.  The step and batched
 // kernels set it for FP32 (kOceanSplit).
-template <typename T, int VAR, int NTRC, int TX, int TY, bool DIAG, bool LATE = false, bool DYN = true,
+template <typename T, int VAR, int NTRC, int TX, int TY, bool DIAG, bool LATE = false, bool ALONE = true,
           bool OSPLIT = false, typename L>
 __device__ __forceinline__ void tile_body(const Dyn<T>& d, const int t, L& lds, const int tid) {
     using S = TileShapeC<TX, TY>;
@@ -1341,12 +1356,12 @@ __device__ __forceinline__ void tile_body(const Dyn<T>& d, const int t, L& lds, 
         if ((tid & 63) == 0) lds.ocean[tid >> 6] = w;
         __syncthreads();
         if (lds.ocean[0] & lds.ocean[1] & lds.ocean[2] & lds.ocean[3])
-            tile_compute<T, VAR, NTRC, TX, TY, DIAG, DYN, true>(d, t, lds, R.g, R.gt, R.eo, R.lo, tid);
+            tile_compute<T, VAR, NTRC, TX, TY, DIAG, ALONE, true>(d, t, lds, R.g, R.gt, R.eo, R.lo, tid);
         else
-            tile_compute<T, VAR, NTRC, TX, TY, DIAG, DYN, false>(d, t, lds, R.g, R.gt, R.eo, R.lo, tid);
+            tile_compute<T, VAR, NTRC, TX, TY, DIAG, ALONE, false>(d, t, lds, R.g, R.gt, R.eo, R.lo, tid);
     } else {
         __syncthreads();
-        tile_compute<T, VAR, NTRC, TX, TY, DIAG, DYN>(d, t, lds, R.g, R.gt, R.eo, R.lo, tid);
+        tile_compute<T, VAR, NTRC, TX, TY, DIAG, ALONE>(d, t, lds, R.g, R.gt, R.eo, R.lo, tid);
     }
 }
 
