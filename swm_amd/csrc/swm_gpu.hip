@@ -2647,7 +2647,7 @@ void swm_gpu_destroy(swm_ctx* c) {
 
 // ---------------------------------------------------------------------------
 // Batched ensembles: contexts attached to one batch advance together, one
-// launch (plus a tiny state-advance launch) per step, replayed from a graph.
+// launch per step, two of them replayed as a graph.
 // ---------------------------------------------------------------------------
 struct swm_batch {
     int fp32 = -1;                       // precision of the members (-1: none attached yet)
@@ -2659,7 +2659,8 @@ struct swm_batch {
     bool on_device = false;              // the device copy is newer than hstep
     bool dirty = true;                   // member list changed since the last build
     void* dmem = nullptr;                // Member<T>[cap]
-    swm::MemberStep* dstep = nullptr;    // MemberStep[cap]
+    swm::MemberStep* dstep = nullptr;    // MemberStep[cap][2]: the current slot of each pair is dstep[2 k + flip]
+    int flip = 0;
     size_t cap = 0;
     int* downer = nullptr;               // member of each work item
     size_t owner_cap = 0;
@@ -2703,8 +2704,11 @@ void batch_drop_graph(swm_batch* b) {
 int batch_pull(swm_batch* b) {
     if (!b->on_device) return 0;
     BHIPCHK(b, hipStreamSynchronize(b->stream));
-    if (!b->hstep.empty())
-        BHIPCHK(b, d2h(b->stream, b->hstep.data(), b->dstep, b->hstep.size() * sizeof(swm::MemberStep)));
+    if (!b->hstep.empty()) {
+        std::vector<swm::MemberStep> pairs(2 * b->hstep.size());
+        BHIPCHK(b, d2h(b->stream, pairs.data(), b->dstep, pairs.size() * sizeof(swm::MemberStep)));
+        for (size_t k = 0; k < b->hstep.size(); ++k) b->hstep[k] = pairs[2 * k + b->flip];
+    }
     b->on_device = false;
     for (size_t k = 0; k < b->mem.size(); ++k) {
         swm_ctx* c = b->mem[k];
@@ -2728,7 +2732,7 @@ int batch_build_t(swm_batch* b) {
         b->cap = 0;
         const size_t cap = std::max<size_t>(n, 2 * b->cap + 16);
         BHIPCHK(b, hipMalloc(&b->dmem, cap * sizeof(swm::Member<T>)));
-        BHIPCHK(b, hipMalloc((void**)&b->dstep, cap * sizeof(swm::MemberStep)));
+        BHIPCHK(b, hipMalloc((void**)&b->dstep, 2 * cap * sizeof(swm::MemberStep)));
         b->cap = cap;
     }
     std::vector<swm::Member<T>> hm(n);
@@ -2766,7 +2770,10 @@ int batch_build_t(swm_batch* b) {
     if (work) BHIPCHK(b, h2d(b->stream, b->downer, owner.data(), (size_t)work * sizeof(int)));
     if (n) {
         BHIPCHK(b, h2d(b->stream, b->dmem, hm.data(), n * sizeof(swm::Member<T>)));
-        BHIPCHK(b, h2d(b->stream, b->dstep, b->hstep.data(), n * sizeof(swm::MemberStep)));
+        std::vector<swm::MemberStep> pairs(2 * n);
+        for (size_t k = 0; k < n; ++k) pairs[2 * k] = pairs[2 * k + 1] = b->hstep[k];
+        BHIPCHK(b, h2d(b->stream, b->dstep, pairs.data(), pairs.size() * sizeof(swm::MemberStep)));
+        b->flip = 0;
     }
     b->on_device = n > 0;
     b->dirty = false;
@@ -2795,11 +2802,11 @@ void batch_launch_k(swm_batch* b, bool queue) {
     if (queue) {
         const int g = std::min(b->nwork, queue_grid<T, V, NT, TX, TY>());
         hipLaunchKernelGGL((swm::batch_queue_kernel<T, V, NT, TX, TY>), dim3(g), dim3(256), 0, b->stream, m,
-                           b->dstep, b->downer, b->nwork, nmem, b->dqueue);
+                           b->dstep + b->flip, b->downer, b->nwork, nmem, b->dqueue);
     } else {
         hipLaunchKernelGGL((swm::batch_kernel<T, V, NT, TX, TY>), dim3(b->nwork), dim3(256), 0, b->stream, m,
-                           b->dstep, b->downer, b->nwork);
-        hipLaunchKernelGGL(swm::batch_advance, dim3((nmem + 255) / 256), dim3(256), 0, b->stream, b->dstep, nmem);
+                           b->dstep + b->flip, b->downer, b->nwork);
+        b->flip ^= 1;
     }
 }
 
@@ -2812,8 +2819,8 @@ void batch_launch_s(swm_batch* b, bool queue) {
     }
 }
 
-// One batched step: the queue kernel's last block advances the members; the
-// one-block-per-tile kernel is followed by batch_advance.
+// One batched step: the queue kernel's last block advances the members in
+// their slots; the one-block-per-tile kernel writes the others, now current.
 template <typename T, int V>
 void batch_launch_v(swm_batch* b) {
     const BatchShape bs = kBatchShapes[b->shape];
@@ -2950,11 +2957,18 @@ int swm_gpu_batch_step(swm_batch* b, int64_t nsteps, int32_t* active) {
         b->last_ms = ms;
         b->on_device = true;
     } else if (!b->mem.empty() && nsteps > 0) {
-        if (!b->graph) {
+        // the graph holds two steps, from slot 0 of the step states back to it;
+        // a step from slot 1 and a last odd one are launched by themselves
+        const int64_t lead = b->flip, pairs = (nsteps - lead) / 2, tail = nsteps - lead - 2 * pairs;
+        if (!b->graph && pairs > 0) {
             HipLock lock(g_hip_mu);
             hipGraph_t g = nullptr;
             BHIPCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
+            const int flip = b->flip;
+            b->flip = 0;
             batch_launch(b);
+            batch_launch(b);
+            b->flip = flip;
             const hipError_t le = hipGetLastError();
             const hipError_t ce = hipStreamEndCapture(b->stream, &g);
             if (le != hipSuccess || ce != hipSuccess) {
@@ -2969,7 +2983,10 @@ int swm_gpu_batch_step(swm_batch* b, int64_t nsteps, int32_t* active) {
             }
         }
         BHIPCHK(b, hipEventRecord(b->ev0, b->stream));
-        for (int64_t k = 0; k < nsteps; ++k) BHIPCHK(b, hipGraphLaunch(b->graph, b->stream));
+        if (lead) batch_launch(b);
+        for (int64_t k = 0; k < pairs; ++k) BHIPCHK(b, hipGraphLaunch(b->graph, b->stream));
+        if (tail) batch_launch(b);
+        BHIPCHK(b, hipGetLastError());
         BHIPCHK(b, hipEventRecord(b->ev1, b->stream));
         BHIPCHK(b, hipEventSynchronize(b->ev1));
         float ms = 0.f;

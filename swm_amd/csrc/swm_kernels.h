@@ -1419,8 +1419,8 @@ step_kernel_p(const Dyn<T> d) {
 // Batched step: many independent domains of uneven size advance by one step in
 // one launch.  Work item w is tile (w - wbase) of member owner[w]; the
 // per-member step state (level, AB ring slot, itt, steps left) lives in
-// device memory and the last block of each step moves it on, so a captured
-// graph of the two launches replays any number of steps.
+// device memory and the step's own launch moves it on, so a captured graph
+// replays any number of steps.
 // ---------------------------------------------------------------------------
 template <typename T>
 struct Member {
@@ -1440,13 +1440,31 @@ struct MemberStep {
     int cur, ring, cbuf, pad;
 };
 
+// Every member has two MemberStep slots, next to each other: a kernel's stp
+// points to the first member's current slot, so member k's is stp[2 k], and the
+// other slot of the pair differs from it in one address bit.
+__device__ __forceinline__ MemberStep* other_slot(const MemberStep* s) {
+    static_assert((sizeof(MemberStep) & (sizeof(MemberStep) - 1)) == 0, "slots pair up by one address bit");
+    return (MemberStep*)((uintptr_t)s ^ sizeof(MemberStep));
+}
+// model_advance of a member that stepped: N0 <- N0p1, G ring moves on.
+__device__ __forceinline__ MemberStep advanced(MemberStep s) {
+    if (s.remaining <= 0) return s;
+    s.itt += 1;
+    s.remaining -= 1;
+    s.cur = 1 - s.cur;
+    s.ring = s.ring == 2 ? 0 : s.ring + 1;
+    s.cbuf = 0;
+    return s;
+}
+
 // Work item w of a batched step: tile (w - wbase) of member owner[w].
 template <typename T, int VAR, int NTRC_MAX, int TX, int TY, typename L>
 __device__ __forceinline__ void batch_item(const Member<T>* __restrict__ mem, const MemberStep* __restrict__ stp,
                                            const int* __restrict__ owner, const int w, L& lds, const int tid) {
     const int lo = owner[w];   // member whose work range holds w
     const Member<T>& m = mem[lo];
-    const MemberStep ms = stp[lo];
+    const MemberStep ms = stp[2 * lo];
     if (ms.remaining <= 0) return;   // whole block: the member is done
     Dyn<T> d{};
     d.s = m.s;
@@ -1477,27 +1495,12 @@ __device__ __forceinline__ void batch_item(const Member<T>* __restrict__ mem, co
     }
 }
 
-// model_advance of every member that stepped: N0 <- N0p1, G ring moves on.
-__device__ __forceinline__ void advance_members(MemberStep* stp, int nmem) {
-    for (int k = threadIdx.x; k < nmem; k += 256) {
-        MemberStep s = stp[k];
-        if (s.remaining <= 0) continue;
-        s.itt += 1;
-        s.remaining -= 1;
-        s.cur = 1 - s.cur;
-        s.ring = s.ring == 2 ? 0 : s.ring + 1;
-        s.cbuf = 0;
-        stp[k] = s;
-    }
-}
-
 // The block that finishes last (device-scope counter ctr[kBatchQueues], fenced)
 // advances every member and clears the step's counters, so one launch is a
 // whole batched step: every other block has read its member's step state
 // before it counted itself done.  Used by the persistent queue kernel, whose
 // grid is the resident blocks; with one block per tile (tens of thousands of
-// blocks) the atomics on one counter serialise and cost more than the
-// separate batch_advance launch.
+// blocks) the atomics on one counter would serialise.
 constexpr int kBatchQueues = 8;
 __device__ __forceinline__ void batch_finish(MemberStep* stp, int nmem, int* ctr) {
     __shared__ int s_last;
@@ -1509,12 +1512,15 @@ __device__ __forceinline__ void batch_finish(MemberStep* stp, int nmem, int* ctr
     __syncthreads();
     if (!s_last) return;
     __threadfence();
-    advance_members(stp, nmem);
+    for (int k = threadIdx.x; k < nmem; k += 256) stp[2 * k] = advanced(stp[2 * k]);
     if (threadIdx.x <= kBatchQueues) ctr[threadIdx.x] = 0;   // tile queues and this counter
 }
 
 // One block per work item; blocks of one XCD take a contiguous run of items
-// (neighbouring tiles of a member share halo lines in that XCD's L2).
+// (neighbouring tiles of a member share halo lines in that XCD's L2).  The block
+// of a member's first tile writes the member's next step state to the slot that
+// no block of this step reads: the launch that did this after each step took
+// 3.9 us of the 56 of a step of 14 members.
 template <typename T, int VAR, int NTRC_MAX, int TX, int TY>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5)))
 batch_kernel(const Member<T>* __restrict__ mem, const MemberStep* __restrict__ stp, const int* __restrict__ owner,
@@ -1523,13 +1529,11 @@ batch_kernel(const Member<T>* __restrict__ mem, const MemberStep* __restrict__ s
     using RTC = RowTabC<TX, TY, NTRC_MAX>;
     __shared__ TileLds<T, NTRC_MAX, (TX + 2) * (TY + 2), TY + 2, 1, DD::DUE, DD::DVE, RTC::LR,
                        RTC::LK> lds;
-    batch_item<T, VAR, NTRC_MAX, TX, TY>(mem, stp, owner, xcd_tile(blockIdx.x, nwork), lds, threadIdx.x);
-}
-
-// model_advance after a batch_kernel step (one thread per member)
-__global__ void __launch_bounds__(256) batch_advance(MemberStep* stp, int nmem) {
-    const int b0 = blockIdx.x * 256;   // this block's members: [b0, b0 + 256)
-    if (b0 < nmem) advance_members(stp + b0, nmem - b0 < 256 ? nmem - b0 : 256);
+    const int w = xcd_tile(blockIdx.x, nwork), k = owner[w];
+    const bool first = w == mem[k].wbase;
+    batch_item<T, VAR, NTRC_MAX, TX, TY>(mem, stp, owner, w, lds, threadIdx.x);
+    // last, so that the loads above stay scalar
+    if (first && threadIdx.x == 0) *other_slot(&stp[2 * k]) = advanced(stp[2 * k]);
 }
 
 // Persistent tile queue: a grid of resident blocks drains the step's work
