@@ -896,11 +896,30 @@ Dyn<T> make_dyn(swm_ctx* c, int tile) {
     return d;
 }
 
+// FULLY_NONLINEAR FP64 domains of more tiles than this split off the all-ocean
+// ones (step_kernel_split): two rounds of the 1280 blocks that are resident at
+// once.  Below, a step is mostly one tile's latency and the longer kernel costs 2
+// to 4 % of it (200^2: 5.50 -> 5.61 us, 512^2 the same); above, it saves mask
+// arithmetic: 1024x768 40.9 -> 40.5 us, 1024^2 with 5 % land and a tracer 38.7 ->
+// 38.1, with no land and two 45.4 -> 42.3, 2304x1800 122.5 -> 116.4, 4096x2048 329
+// -> 316.
+constexpr int kSplitTiles = 2560;
+
 template <typename T, int TX, int TY, bool DIAG, bool LATE = false>
 void launch_tile(swm_ctx* c, const Dyn<T>& d) {
     const int var = c->d.variant;
     const int nt = (int)c->trc.size();
     dim3 grid(d.nblk), block(256);
+    if constexpr (sizeof(T) == 8 && !DIAG && TX == 32 && TY == 8 && LATE)
+        if (var == SWM_FULLY_NONLINEAR && d.nblk > kSplitTiles) {
+#define SWM_LAUNCH(N)                                                                                                 \
+    hipLaunchKernelGGL((swm::step_kernel_split<T, swm::VAR_FN, N, TX, TY, LATE>), grid, block, 0, c->stream, d)
+            if (nt == 0) SWM_LAUNCH(0);
+            else if (nt == 1) SWM_LAUNCH(1);
+            else SWM_LAUNCH(2);
+#undef SWM_LAUNCH
+            return;
+        }
 #define SWM_LAUNCH(V, N) \
     hipLaunchKernelGGL((swm::step_kernel<T, V, N, TX, TY, DIAG, LATE>), grid, block, 0, c->stream, d)
     if (var == SWM_LINEARISED_MEAN_STATE) {   // no tracers on the linear variants

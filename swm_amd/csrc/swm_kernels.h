@@ -1312,8 +1312,8 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
 // tile_body): FP32 only.  On the 1024^2 basin with 5 % islands 70 % of the
 // 32x8 tiles are all ocean, and the FP32 step is 6 % faster (31.7 -> 29.8 us).
 // FP64 takes 96 VGPRs with both instantiations in one kernel (80 with one) and
-// gains 2 to 4 % from 1024^2 on, but the longer kernel costs 2 to 4 % of the 5 to
-// 8 us of a small grid's step.
+// gains 2 to 7 % from 1024^2 on, but the longer kernel costs 2 to 4 % of the 5 to
+// 8 us of a small grid's step: a kernel of its own takes the large ones.
 template <typename T>
 inline constexpr bool kOceanSplit = sizeof(T) == 4;
 
@@ -1373,6 +1373,19 @@ step_kernel(const Dyn<T> d) {
     __shared__ TileLds<T, NTRC, (TX + 2) * (TY + 2), TY + 2,
                        (VAR == VAR_MS ? (TX + 2) * (TY + 2) : 1), DD::DUE, DD::DVE, RTC::LR, RTC::LK> lds;
     tile_body<T, VAR, NTRC, TX, TY, DIAG, LATE, true, kOceanSplit<T>>(d, xcd_tile(blockIdx.x, d.nblk), lds, threadIdx.x);
+}
+
+// step_kernel with the all-ocean tiles split off, for FP64 domains of many tiles:
+// bound by vector issue as much as by memory, they gain from the mask arithmetic
+// that such tiles leave out.
+template <typename T, int VAR, int NTRC, int TX, int TY, bool LATE>
+__global__ void __launch_bounds__(256)
+step_kernel_split(const Dyn<T> d) {
+    using DD = LdsDuDv<T, TX, TY>;
+    using RTC = RowTabC<TX, TY, NTRC>;
+    __shared__ TileLds<T, NTRC, (TX + 2) * (TY + 2), TY + 2,
+                       (VAR == VAR_MS ? (TX + 2) * (TY + 2) : 1), DD::DUE, DD::DVE, RTC::LR, RTC::LK> lds;
+    tile_body<T, VAR, NTRC, TX, TY, false, LATE, true, true>(d, xcd_tile(blockIdx.x, d.nblk), lds, threadIdx.x);
 }
 
 // Persistent tile kernel: block b advances the tiles [b*tpb, (b+1)*tpb) in
