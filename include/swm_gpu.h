@@ -299,8 +299,8 @@ int swm_gpu_sums_noalloc(swm_ctx *c, int32_t tracer_id, double *out);
  * without oscillating forcing.  Each batch step is one launch covering every
  * tile of every attached member (SWM_timestep + TRC_timestep + model_advance
  * per member, the same arithmetic as swm_gpu_step, so a member's result is the
- * same alone and in the batch) plus a launch that moves the members' step
- * state on; the pair is captured once in a hipGraph and replayed.
+ * same alone and in the batch), which also moves the members' step state on;
+ * two steps are captured once in a hipGraph and replayed.
  *   attach:    the context joins and will advance nsteps more steps; while
  *              attached, swm_gpu_step / upload_state / add_tracer on it fail,
  *              and sync / sums / divergence / itt see its current state.
