@@ -902,7 +902,9 @@ Dyn<T> make_dyn(swm_ctx* c, int tile) {
 // to 4 % of it (200^2: 5.50 -> 5.61 us, 512^2 the same); above, it saves mask
 // arithmetic: 1024x768 40.9 -> 40.5 us, 1024^2 with 5 % land and a tracer 38.7 ->
 // 38.1, with no land and two 45.4 -> 42.3, 2304x1800 122.5 -> 116.4, 4096x2048 329
-// -> 316.
+// -> 316.  FP64 batches take the same line (batch_kernel_split): 14 members of 8856
+// tiles 92.0 -> 87.8 us a step, 30 of 34165 315 -> 299, 40 small ones of 5530 the
+// same within 1 %; below it the split cost 4 members of 163 tiles 1.4 %.
 constexpr int kSplitTiles = 2560;
 
 template <typename T, int TX, int TY, bool DIAG, bool LATE = false>
@@ -2823,8 +2825,16 @@ void batch_launch_k(swm_batch* b, bool queue) {
         hipLaunchKernelGGL((swm::batch_queue_kernel<T, V, NT, TX, TY>), dim3(g), dim3(256), 0, b->stream, m,
                            b->dstep + b->flip, b->downer, b->nwork, nmem, b->dqueue);
     } else {
-        hipLaunchKernelGGL((swm::batch_kernel<T, V, NT, TX, TY>), dim3(b->nwork), dim3(256), 0, b->stream, m,
-                           b->dstep + b->flip, b->downer, b->nwork);
+        bool split = false;   // by the same line as a domain stepped alone
+        if constexpr (sizeof(T) == 8 && V == swm::VAR_FN && TX == 32) {
+            split = b->nwork > kSplitTiles;
+            if (split)
+                hipLaunchKernelGGL((swm::batch_kernel_split<T, V, NT, TX, TY>), dim3(b->nwork), dim3(256), 0,
+                                   b->stream, m, b->dstep + b->flip, b->downer, b->nwork);
+        }
+        if (!split)
+            hipLaunchKernelGGL((swm::batch_kernel<T, V, NT, TX, TY>), dim3(b->nwork), dim3(256), 0, b->stream, m,
+                               b->dstep + b->flip, b->downer, b->nwork);
         b->flip ^= 1;
     }
 }

@@ -1472,7 +1472,7 @@ __device__ __forceinline__ MemberStep advanced(MemberStep s) {
 }
 
 // Work item w of a batched step: tile (w - wbase) of member owner[w].
-template <typename T, int VAR, int NTRC_MAX, int TX, int TY, typename L>
+template <typename T, int VAR, int NTRC_MAX, int TX, int TY, bool SPLIT = kOceanSplit<T>, typename L>
 __device__ __forceinline__ void batch_item(const Member<T>* __restrict__ mem, const MemberStep* __restrict__ stp,
                                            const int* __restrict__ owner, const int w, L& lds, const int tid) {
     const int lo = owner[w];   // member whose work range holds w
@@ -1497,14 +1497,14 @@ __device__ __forceinline__ void batch_item(const Member<T>* __restrict__ mem, co
     d.dtc3 = m.dtc[tstep - 1][2];
     const int t = w - m.wbase;
     if constexpr (NTRC_MAX == 0) {
-        tile_body<T, VAR, 0, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds, tid);
+        tile_body<T, VAR, 0, TX, TY, false, false, false, SPLIT>(d, t, lds, tid);
     } else if constexpr (NTRC_MAX == 1) {
-        if (m.ntr == 0) tile_body<T, VAR, 0, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds, tid);
-        else tile_body<T, VAR, 1, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds, tid);
+        if (m.ntr == 0) tile_body<T, VAR, 0, TX, TY, false, false, false, SPLIT>(d, t, lds, tid);
+        else tile_body<T, VAR, 1, TX, TY, false, false, false, SPLIT>(d, t, lds, tid);
     } else {
-        if (m.ntr == 0) tile_body<T, VAR, 0, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds, tid);
-        else if (m.ntr == 1) tile_body<T, VAR, 1, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds, tid);
-        else tile_body<T, VAR, 2, TX, TY, false, false, false, kOceanSplit<T>>(d, t, lds, tid);
+        if (m.ntr == 0) tile_body<T, VAR, 0, TX, TY, false, false, false, SPLIT>(d, t, lds, tid);
+        else if (m.ntr == 1) tile_body<T, VAR, 1, TX, TY, false, false, false, SPLIT>(d, t, lds, tid);
+        else tile_body<T, VAR, 2, TX, TY, false, false, false, SPLIT>(d, t, lds, tid);
     }
 }
 
@@ -1529,11 +1529,21 @@ __device__ __forceinline__ void batch_finish(MemberStep* stp, int nmem, int* ctr
     if (threadIdx.x <= kBatchQueues) ctr[threadIdx.x] = 0;   // tile queues and this counter
 }
 
+// Work item w and, in the block of a member's first tile, the member's next step
+// state into the slot that no block of this step reads: the launch that did this
+// after each step took 3.9 us of the 56 of a step of 14 members.
+template <typename T, int VAR, int NTRC_MAX, int TX, int TY, bool SPLIT, typename L>
+__device__ __forceinline__ void batch_block(const Member<T>* __restrict__ mem, const MemberStep* __restrict__ stp,
+                                            const int* __restrict__ owner, const int w, L& lds) {
+    const int k = owner[w];
+    const bool first = w == mem[k].wbase;
+    batch_item<T, VAR, NTRC_MAX, TX, TY, SPLIT>(mem, stp, owner, w, lds, threadIdx.x);
+    // last, so that the loads above stay scalar
+    if (first && threadIdx.x == 0) *other_slot(&stp[2 * k]) = advanced(stp[2 * k]);
+}
+
 // One block per work item; blocks of one XCD take a contiguous run of items
-// (neighbouring tiles of a member share halo lines in that XCD's L2).  The block
-// of a member's first tile writes the member's next step state to the slot that
-// no block of this step reads: the launch that did this after each step took
-// 3.9 us of the 56 of a step of 14 members.
+// (neighbouring tiles of a member share halo lines in that XCD's L2).
 template <typename T, int VAR, int NTRC_MAX, int TX, int TY>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5)))
 batch_kernel(const Member<T>* __restrict__ mem, const MemberStep* __restrict__ stp, const int* __restrict__ owner,
@@ -1542,11 +1552,20 @@ batch_kernel(const Member<T>* __restrict__ mem, const MemberStep* __restrict__ s
     using RTC = RowTabC<TX, TY, NTRC_MAX>;
     __shared__ TileLds<T, NTRC_MAX, (TX + 2) * (TY + 2), TY + 2, 1, DD::DUE, DD::DVE, RTC::LR,
                        RTC::LK> lds;
-    const int w = xcd_tile(blockIdx.x, nwork), k = owner[w];
-    const bool first = w == mem[k].wbase;
-    batch_item<T, VAR, NTRC_MAX, TX, TY>(mem, stp, owner, w, lds, threadIdx.x);
-    // last, so that the loads above stay scalar
-    if (first && threadIdx.x == 0) *other_slot(&stp[2 * k]) = advanced(stp[2 * k]);
+    batch_block<T, VAR, NTRC_MAX, TX, TY, kOceanSplit<T>>(mem, stp, owner, xcd_tile(blockIdx.x, nwork), lds);
+}
+
+// batch_kernel with the all-ocean tiles split off, for FP64 batches of many
+// tiles (as step_kernel_split).
+template <typename T, int VAR, int NTRC_MAX, int TX, int TY>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5)))
+batch_kernel_split(const Member<T>* __restrict__ mem, const MemberStep* __restrict__ stp,
+                   const int* __restrict__ owner, int nwork) {
+    using DD = LdsDuDv<T, TX, TY>;
+    using RTC = RowTabC<TX, TY, NTRC_MAX>;
+    __shared__ TileLds<T, NTRC_MAX, (TX + 2) * (TY + 2), TY + 2, 1, DD::DUE, DD::DVE, RTC::LR,
+                       RTC::LK> lds;
+    batch_block<T, VAR, NTRC_MAX, TX, TY, true>(mem, stp, owner, xcd_tile(blockIdx.x, nwork), lds);
 }
 
 // Persistent tile queue: a grid of resident blocks drains the step's work
