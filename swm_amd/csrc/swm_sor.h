@@ -101,29 +101,30 @@ __device__ __forceinline__ double keep(double c, int m) {
     return __longlong_as_double(((long long)((int)(b >> 32) & m) << 32) | (unsigned)((int)b & m));
 }
 __device__ __forceinline__ float keep(float c, int m) { return __int_as_float(__float_as_int(c) & m); }
-// m ? a : b with the lane mask m in a scalar register pair (the 64-bit
-// encoding): the 32-bit encoding, which reads vcc, holds a wavefront up for
-// some 19 cycles when two of them follow each other, as a double's two halves
-// do; this one takes 4.
-__device__ __forceinline__ int sel(unsigned long long m, int a, int b) {
-    int d;
-    asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(d) : "v"(b), "v"(a), "s"(m));
-    return d;
-}
-__device__ __forceinline__ double sel(unsigned long long m, double a, double b) {
-    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
-    const int lo = sel(m, (int)x, (int)y), hi = sel(m, (int)(x >> 32), (int)(y >> 32));
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-__device__ __forceinline__ double dvr_e64(double a, double b, double y) {   // dvr
+// dvr with its last choice, q0 where it is zero or infinite, made through a lane
+// mask in a scalar register pair by the selects' 64-bit encoding: the 32-bit
+// one, which reads vcc, holds a wavefront up for some 19 cycles when two of them
+// follow each other, as a double's two halves do; this one takes 4.
+// A vector instruction may read a scalar register that another one wrote only two
+// wait states later.  The compiler keeps that distance in its own code but not
+// between asm statements, so the mask is written and read in one (2048 x 1024
+// FP64, a solve of 5000 sweeps: 34.9 ms, and 34.8 with other instructions there).
+__device__ __forceinline__ double dvr_e64(double a, double b, double y) {
     const double q0 = a * y;
     double r = __builtin_fma(-b, q0, a);
     const double q1 = __builtin_fma(r, y, q0);
     r = __builtin_fma(-b, q1, a);
     const double q2 = __builtin_fma(r, y, q1);
+    const long long x = __double_as_longlong(q0), z = __double_as_longlong(q2);
+    int lo = (int)z, hi = (int)(z >> 32);
     unsigned long long m;
-    asm("v_cmp_class_f64_e64 %0, %1, %2" : "=s"(m) : "v"(q0), "s"(0x264));
-    return sel(m, q0, q2);
+    asm("v_cmp_class_f64_e64 %0, %3, %6\n\t"
+        "s_nop 1\n\t"
+        "v_cndmask_b32_e64 %1, %1, %4, %0\n\t"
+        "v_cndmask_b32_e64 %2, %2, %5, %0"
+        : "=&s"(m), "+&v"(lo), "+&v"(hi)
+        : "v"(q0), "v"((int)x), "v"((int)(x >> 32)), "s"(0x264));   // 0x264: -inf, -0, +0, +inf
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 __device__ __forceinline__ float dvr_e64(float a, float b, float y) { return a * y; }
 // value of the lane to the left (wave_shr:1) / right (wave_shl:1), 0 at the wavefront's ends
