@@ -989,8 +989,10 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
         // integrate_AB (src/time_integration_module.f90:74-112) of one field: x plus
         // the increments of its history g0, g1 and the new tendency, over the
         // implicit damping.  FP64 divides by the row's divisor through its
-        // reciprocal; FP32 statics hold 1 - 1/impl, and the increments are added to
-        // the carried pair (x, lo_in).
+        // reciprocal, and by a full array's as written (a reciprocal formed here
+        // would cost the same division and miss the last place below 1e-300); FP32
+        // statics hold 1 - 1/impl, and the increments are added to the carried pair
+        // (x, lo_in).
         auto ab = [&](T x, T g0, T g1, T g2, unsigned short lo_in, unsigned full, auto& f, bool ocean, int e, int er,
                       unsigned short& lo) -> T {
             T b = rvs(ocean, e, e + 1);
@@ -1001,15 +1003,13 @@ __device__ __forceinline__ void tile_compute(const Dyn<T>& d, const int t, L& ld
                 if (d.tstep >= 3) inc = madd(inc, d.dtc3, g2);
                 return carry_step(x, lo_in, inc, b, lo);
             } else {
-                T y = rvs(ocean, er, er + 1);
-                if (opt & full) {
-                    b = gld(f.full, off);
-                    y = T(1) / b;
-                }
+                const T y = rvs(ocean, er, er + 1);
                 x = madd(x, d.dtc1, g0);
                 if (d.tstep >= 2) x = madd(x, d.dtc2, g1);
                 if (d.tstep >= 3) x = madd(x, d.dtc3, g2);
-                return dvr(x, b, y);
+                T r = dvr(x, b, y);
+                if (opt & full) r = dv(x, gld(f.full, off));
+                return r;
             }
         };
         // the sections below are scheduled one after another, which keeps each
