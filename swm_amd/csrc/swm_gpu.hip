@@ -8,6 +8,8 @@
 // time step (steady-state cycles replayed as HIP graphs).
 #include <hip/hip_runtime.h>
 
+#include <sched.h>
+
 #include <algorithm>
 #include <cmath>
 #include <condition_variable>
@@ -16,6 +18,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <type_traits>
@@ -374,18 +377,94 @@ hipError_t h2d_rows(hipStream_t s, void* dst, size_t dpitch, const void* src, si
     return e;
 }
 
-// A device plane of S, with its bfloat16 low part if lo is given (pitch c->P
-// both), as host doubles dst[Ny][Nx] = f(value, low part's bits), in stream order.  The plane comes in pieces of about kPiece bytes, all enqueued
-// at once; the host unpacks one while the next is on its way.  From kThreaded
-// bytes on, kHostThreads - 1 threads that live for the call unpack too: there
-// it is mostly first touches of the caller's pages.  Only the calling thread
-// calls HIP.  Against one transfer, one thread and, for FP32, a copy to convert
-// from: 0.41 -> 0.33 ms a 1024^2 field in FP64 and 0.50 -> 0.25 in FP32, 1.93 ->
-// 0.90 at 2304x1800 in FP64; a 96x64 field costs the same 14 us.  Pieces of 256
-// KiB are slower (2304x1800: the same, 1024x768: 0.39 -> 0.65 ms a field), more
-// threads and threads below 4 MB not faster (487x333: 0.045 -> 0.06 ms a field).
-constexpr size_t kPiece = (size_t)1 << 20, kThreaded = (size_t)4 << 20;
+// Threads that help to unpack fields: of the library, like the staging buffer,
+// and like it used under g_hip_mu, so for one field at a time.  They start with
+// the first field that wants them, sleep between fields and end with the last
+// context.  The calling thread takes pieces too and waits for none but those a
+// thread has taken: on a host whose CPUs are busy (BLAS threads spin on for
+// a while after a call) a thread that was just woken can stay off them for a
+// scheduler tick of 4 ms, and what it has not begun is done without it.  Waiting
+// for the threads themselves cost 4 ms a field there (1024^2: 4.0 -> 0.45 ms).
 constexpr int kHostThreads = 4;
+struct Unpackers {
+    std::mutex mu;
+    std::condition_variable wake, idle;
+    std::vector<std::thread> th;
+    void (*run)(void*, size_t) = nullptr;   // the field's unpack(arg, piece)
+    void* arg = nullptr;
+    size_t here = 0, next = 0;   // pieces that have arrived, and that a thread has taken
+    int busy = 0;                // threads at work on a piece
+    bool stop = false;
+
+    Unpackers() {
+        cpu_set_t cpus;
+        const int n = sched_getaffinity(0, sizeof(cpus), &cpus) == 0 ? CPU_COUNT(&cpus) : 1;
+        try {
+            th.reserve(kHostThreads);
+            while ((int)th.size() < std::min(n, kHostThreads) - 1) th.emplace_back([this] { work(); });
+        } catch (...) {   // fewer threads: the caller takes what they would have
+        }
+    }
+    ~Unpackers() {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            stop = true;
+        }
+        wake.notify_all();
+        for (auto& t : th) t.join();
+    }
+    void work() {
+        for (std::unique_lock<std::mutex> lk(mu);;) {
+            wake.wait(lk, [this] { return stop || next < here; });
+            if (stop) return;
+            take(lk);
+        }
+    }
+    void take(std::unique_lock<std::mutex>& lk) {
+        const size_t p = next++;
+        ++busy;
+        lk.unlock();
+        run(arg, p);
+        lk.lock();
+        if (--busy == 0) idle.notify_one();
+    }
+    void begin(void (*f)(void*, size_t), void* a) {
+        std::lock_guard<std::mutex> lk(mu);
+        run = f;
+        arg = a;
+        here = next = 0;
+    }
+    // One more piece has arrived.  The caller does one itself where pieces pile up
+    // though not every thread is at work, and else goes on to announce the next.
+    void arrived() {
+        std::unique_lock<std::mutex> lk(mu);
+        ++here;
+        wake.notify_one();
+        if (th.empty() || (here - next > 1 && busy < (int)th.size())) take(lk);
+    }
+    // Returns with no piece left and no thread at work; cancel: with those begun done.
+    void finish(bool cancel) {
+        std::unique_lock<std::mutex> lk(mu);
+        if (cancel) next = here;
+        while (next < here) take(lk);
+        idle.wait(lk, [this] { return busy == 0; });
+    }
+};
+Unpackers* g_unpackers = nullptr;
+int g_contexts = 0;
+
+// A device plane of S, with its bfloat16 low part if lo is given (pitch c->P
+// both), as host doubles dst[Ny][Nx] = f(value, low part's bits), in stream
+// order.  The plane comes in pieces of about kPiece bytes, all enqueued at once;
+// the host unpacks one while the next is on its way.  From kThreaded bytes on
+// the Unpackers help: there it is mostly first touches of the caller's pages.
+// Only the calling thread calls HIP.  Against one transfer, one thread and, for
+// FP32, a copy to convert from: 0.41 -> 0.33 ms a 1024^2 field in FP64 and 0.50 ->
+// 0.25 in FP32, 1.93 -> 0.90 at 2304x1800 in FP64; a 96x64 field costs the same
+// 14 us.  Pieces of 256 KiB are slower (2304x1800: the same, 1024x768: 0.39 ->
+// 0.65 ms a field), more threads and threads below 4 MB not faster (487x333:
+// 0.045 -> 0.06 ms a field).
+constexpr size_t kPiece = (size_t)1 << 20, kThreaded = (size_t)4 << 20;
 template <typename S, typename F>
 hipError_t plane_to_host(swm_ctx* c, double* dst, const void* src, const void* lo, F f) {
     constexpr size_t kMaxPieces = sizeof(c->ev_piece) / sizeof(c->ev_piece[0]);
@@ -427,42 +506,21 @@ hipError_t plane_to_host(swm_ctx* c, double* dst, const void* src, const void* l
                     for (size_t i = 0; i < Nx; ++i) out[i] = f(in[i], 0);
             }
         };
-        std::mutex mu;
-        std::condition_variable cv;
-        size_t here = 0, next = 0;   // pieces that have arrived, and that a thread has taken
-        bool failed = false;
-        auto work = [&] {
-            for (std::unique_lock<std::mutex> lk(mu);;) {
-                cv.wait(lk, [&] { return failed || next < here || next == np; });
-                if (failed || next == np) return;
-                const size_t p = next++;
-                if (next == np) cv.notify_all();
-                lk.unlock();
-                unpack(p);
-                lk.lock();
-            }
-        };
-        std::thread th[kHostThreads - 1];
-        if (nr * Nx * sizeof(double) >= kThreaded) try {
-                for (size_t w = 0; w + 1 < std::min<size_t>(kHostThreads, np); ++w) th[w] = std::thread(work);
-            } catch (...) {   // fewer threads: this one takes what they would have
-            }
+        Unpackers* help = nullptr;
+        if (nr * Nx * sizeof(double) >= kThreaded) {
+            if (!g_unpackers) g_unpackers = new (std::nothrow) Unpackers;
+            help = g_unpackers;
+        }
+        if (help) {
+            help->begin([](void* u, size_t p) { (*(decltype(unpack)*)u)(p); }, &unpack);
+        }
         for (size_t p = 0; p < np && e == hipSuccess; ++p) {
             e = np > 1 ? hipEventSynchronize(c->ev_piece[p]) : hipStreamSynchronize(c->stream);
-            {
-                std::lock_guard<std::mutex> lk(mu);
-                if (e == hipSuccess) here = p + 1; else failed = true;
-            }
-            cv.notify_one();
-            if (!th[0].joinable() && e == hipSuccess) {
-                next = p + 1;
-                unpack(p);
-            }
+            if (e != hipSuccess) break;
+            if (help) help->arrived();
+            else unpack(p);
         }
-        if (e != hipSuccess) cv.notify_all();
-        if (e == hipSuccess) work();
-        for (auto& t : th)
-            if (t.joinable()) t.join();
+        if (help) help->finish(e != hipSuccess);
     }
     return e;
 }
@@ -1271,6 +1329,7 @@ int swm_gpu_create(const swm_desc* d, swm_ctx** out) {
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) { g_create_err = "no HIP device"; return 5; }
     swm_ctx* c = new swm_ctx();
+    ++g_contexts;
     const int rc = create_impl(c, d);
     if (rc) {
         g_create_err = c->err.empty() ? "create failed" : c->err;
@@ -2662,6 +2721,10 @@ void swm_gpu_destroy(swm_ctx* c) {
         if (e) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
+    if (--g_contexts == 0) {
+        delete g_unpackers;
+        g_unpackers = nullptr;
+    }
 }
 
 }  // extern "C"
