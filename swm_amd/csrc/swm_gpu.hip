@@ -521,6 +521,7 @@ hipError_t plane_to_host(swm_ctx* c, double* dst, const void* src, const void* l
             else unpack(p);
         }
         if (help) help->finish(e != hipSuccess);
+        if (e != hipSuccess) (void)hipStreamSynchronize(c->stream);   // as above
     }
     return e;
 }

@@ -94,3 +94,21 @@ os.sched_setaffinity(0, {min(os.sched_getaffinity(0))})
 assert np.array_equal(g.get("SWM_U"), u)
 assert threads() == before
 """)
+
+
+@pytest.mark.parametrize("nx", [800, 300])
+def test_failed_wait_leaves_no_copy_into_the_staging_buffer(host_hip, nx):
+    """The staging buffer is the next transfer's: a read whose wait for a piece
+    fails returns only when the pieces still on their way have landed."""
+    run(host_hip, """
+u, g = context(%d)
+assert np.array_equal(g.get("SWM_U"), u)
+hip.host_hip_fail_event(2)
+try:
+    g.get("SWM_U")
+    raise SystemExit("no error")
+except gpu.SwmGpuError as e:
+    assert "injected" in str(e)
+assert hip.host_hip_copies_open() == 0
+assert np.array_equal(g.get("SWM_U"), u)
+""" % nx)
