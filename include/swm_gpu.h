@@ -231,10 +231,10 @@ int swm_gpu_avg_read(swm_ctx *c, int32_t avg_id, double *host_out, double *weigh
  * launch per colour, -1 (default) for four sweeps per launch whatever the
  * cadence (any sweep of a launch can be a tested one and the one that passes).
  * Grids with an odd extent that is open across its periodic seam take, for -1,
- * the largest of 4, 2, 1 sweeps that divides the cadence.  The reference mode
- * (test after every sweep) uses K = halo / 2 sweeps per launch, 4 for halo -1,
- * and one launch per colour for halo 0.  Every halo gives the same chi bit for
- * bit and the same sweep count. */
+ * two sweeps per launch, or one where the cadence is odd.  The reference mode
+ * (test after every sweep) uses K = halo / 2 sweeps per launch, for halo -1 four
+ * (two on grids open at an odd seam), and one launch per colour for halo 0.  Every
+ * halo gives the same chi bit for bit and the same sweep count. */
 int swm_gpu_kernel_shape_count(void);
 int swm_gpu_set_kernel_shape(swm_ctx *c, int32_t shape);
 int swm_gpu_tune(swm_ctx *c, int32_t steps, int32_t *best_shape, double *times_ms);
@@ -243,8 +243,8 @@ int swm_gpu_launch_mode(const swm_ctx *c, int32_t *graphs, double *ms_direct, do
 int swm_gpu_set_sor_check_every(swm_ctx *c, int32_t every);
 int swm_gpu_set_sor_halo(swm_ctx *c, int32_t halo);
 /* rows of the 64-column LDS tile of grids with an odd extent that is open
- * across its periodic seam: 16 (default) or 32 (fewer halo cells per output;
- * not with the 8-cell halo, whose 64x32 tile would exceed 64 KiB of LDS).
+ * across its periodic seam: 16 (default) or 32 (fewer halo cells per output; 24
+ * rows with two sweeps per launch, within 64 KiB of LDS; not with the 8-cell halo).
  * Other grids choose their tile by their size.  Every tile gives the same chi
  * bit for bit. */
 int swm_gpu_set_sor_tile_rows(swm_ctx *c, int32_t rows);

@@ -1726,9 +1726,10 @@ namespace {
 // the sweep precision, coefficient tables in that precision, the omega schedule.
 int sor_prepare(swm_ctx* c, bool f32, int nblk) {
     if (!c->sor_partial) {
-        // partial sums of the colour launches (2 x nblk) or of the blocked
-        // sweeps (one per 64 x 16 tile, two sets by launch parity)
-        const size_t nb = std::max<size_t>(2 * (size_t)nblk, 2 * (size_t)((c->Nx + 63) / 64) * ((c->Ny + 15) / 16));
+        // partial sums of the colour launches (2 x nblk, and one for a seam's
+        // cells) or of the blocked sweeps (one per 64 x 16 tile, two sets by
+        // launch parity)
+        const size_t nb = std::max<size_t>(2 * ((size_t)nblk + 1), 2 * (size_t)((c->Nx + 63) / 64) * ((c->Ny + 15) / 16));
         c->sor_partial = (double*)dalloc(c, sizeof(double) * nb);
         c->sor_done = (int*)dalloc(c, sizeof(int));
         c->sor_iters = (long long*)dalloc(c, sizeof(long long));
@@ -1777,11 +1778,14 @@ int sor_prepare(swm_ctx* c, bool f32, int nblk) {
     return 0;
 }
 
-// Whether the two colours alternate everywhere a sweep couples cells: even
+// 0 where the two colours alternate everywhere a sweep couples cells: even
 // extents, or odd ones with no ocean face across their periodic seam (every
-// closed basin).  sor_rows needs it; other grids take sor_block.
-bool sor_regular(const swm_ctx* c) {
-    return (c->Nx % 2 == 0 || c->sor_closed_x) && (c->Ny % 2 == 0 || c->sor_closed_y);
+// closed basin); sor_rows takes these grids.  Of the others, which sor_block and
+// the colour launches sweep in the seam's order (swm::sor_late), the odd
+// extents: bit 0 x, bit 1 y.
+int sor_seam_bits(const swm_ctx* c) {
+    const bool open = (c->Nx % 2 && !c->sor_closed_x) || (c->Ny % 2 && !c->sor_closed_y);
+    return open ? c->Nx % 2 | c->Ny % 2 << 1 : 0;
 }
 
 // Buffers and tables of sor_rows, made on first use and kept: the coefficient
@@ -1950,7 +1954,7 @@ void sor_block_launch(swm_ctx* c, const void* chi_in, void* chi_out, void* dB, v
     const int ntx = (c->Nx + TX - 1) / TX;
     const int nb = ntx * ((c->Ny + TY - 1) / TY);
     swm::SorArgs<T> a{};
-    a.Nx = c->Nx; a.Ny = c->Ny; a.P = c->P; a.color = 0; a.sweep = (int)l;
+    a.Nx = c->Nx; a.Ny = c->Ny; a.P = c->P; a.color = 0; a.sweep = (int)l; a.seam = sor_seam_bits(c);
     a.chi = nullptr; a.B = (const T*)dB; a.mask = c->mask;
     a.relax = ref_mode ? (const double*)c->sor_relax : nullptr;
     a.nrelax = c->sor_nrelax; a.omega = omega;
@@ -1987,7 +1991,8 @@ int sor_sweeps(swm_ctx* c, void* dchi, void* dB, void* const* tabs, bool ref_mod
                       double bnorm, int64_t max_sweeps, int nblk, int* host_done) {
     const int every = ref_mode ? 1 : c->sor_every;   // the reference tests after every sweep
     *host_done = 0;
-    if (c->sor_blocked && c->sor_halo != 0 && sor_regular(c))
+    const int seam = sor_seam_bits(c);
+    if (c->sor_blocked && c->sor_halo != 0 && !seam)
         return sor_rows_sweeps<T>(c, dchi, dB, ref_mode, omega, tol, bnorm, max_sweeps, every,
                                   c->sor_halo < 0 ? 4 : c->sor_halo / 2, host_done);
     // sweeps enqueued between reads of the convergence flag: 32 at first (a
@@ -1996,21 +2001,20 @@ int sor_sweeps(swm_ctx* c, void* dchi, void* dB, void* const* tabs, bool ref_mod
     int64_t batch = std::max(32, 4 * every);
     const int64_t batch_max = std::max(256, 4 * every);
     int64_t l = 1;
-    // Blocked sweeps, chi alternating between dchi and the second buffer: K = 4
-    // or 2 sweeps per launch in fixed-omega mode when the test cadence is a
-    // multiple of it, else (and in the reference mode, which tests every sweep
-    // with its Chebyshev omega) one sweep per launch.
-    // sweeps per launch K: a set halo (2K cells), else the largest of 4, 2, 1
-    // that divides the test cadence; the reference mode tests every sweep (K <= 1)
-    int K = c->sor_halo >= 0 ? c->sor_halo / 2 : (every % 4 == 0 ? 4 : (every % 2 == 0 ? 2 : 1));
-    // the reference mode tests every sweep: a launch of K > 1 sweeps keeps the
-    // chi and residual of its first K - 1 sweeps too (mid); K from the halo,
-    // 4 by default
-    if (ref_mode) K = c->sor_halo < 0 ? 4 : c->sor_halo / 2;
+    // Blocked sweeps, chi alternating between dchi and the second buffer, K to a
+    // launch: a set halo's (2K cells), else two, or one where the fixed-omega test
+    // cadence is odd (us a sweep with K = 4, 2, 1 and one colour per launch: 45, 27,
+    // 29, 51 at 2047 x 1024 FP64, 13.4, 9.8, 12.1, 19 at 721 x 361).  The reference
+    // mode tests every sweep with its Chebyshev omega: a launch of K > 1 sweeps
+    // keeps the chi and residual of its first K - 1 sweeps too (mid).
+    int K = c->sor_halo >= 0 ? c->sor_halo / 2 : ref_mode || every % 2 == 0 ? 2 : 1;
     if (!c->sor_blocked) K = 0;
+    // an odd extent narrower than the tile's halo has its seam there more than once
+    if (((seam & 1) && c->Nx < 2 * K + 2) || ((seam & 2) && c->Ny < 2 * K + 2)) K = 0;
     const bool mid = ref_mode && K > 1;
     if (!ref_mode && K > 1 && every % K) return fail(c, "the SOR halo's sweeps per launch must divide the test cadence", 1);
-    const int rows = (K == 4) ? 16 : c->sor_rows;   // 64x32 tiles with a 4-sweep halo exceed 64 KiB of LDS
+    // within 64 KiB of LDS: 16-row tiles with four sweeps, up to 24 rows with two, 32 with one
+    const int rows = K == 4 || c->sor_rows == 16 ? 16 : K == 2 ? 24 : 32;
     if (mid) {
         const int w = std::is_same<T, float>::value ? 1 : 0;
         const size_t bytes = (size_t)c->P * c->Ny * sizeof(T);
@@ -2044,7 +2048,7 @@ int sor_sweeps(swm_ctx* c, void* dchi, void* dB, void* const* tabs, bool ref_mod
                 const bool check = ((l + K - 1) % every) == 0 || l + K - 1 == max_sweeps;
                 const int par = (int)(n & 1);
                 if (K == 4) sor_block_launch<T, 4, 16>(c, cur, alt, dB, tabs, omega, tol, bnorm, l, check, ref_mode, par, pending, mid);
-                else if (K == 2 && rows == 32) sor_block_launch<T, 2, 32>(c, cur, alt, dB, tabs, omega, tol, bnorm, l, check, ref_mode, par, pending, mid);
+                else if (K == 2 && rows == 24) sor_block_launch<T, 2, 24>(c, cur, alt, dB, tabs, omega, tol, bnorm, l, check, ref_mode, par, pending, mid);
                 else if (K == 2) sor_block_launch<T, 2, 16>(c, cur, alt, dB, tabs, omega, tol, bnorm, l, check, ref_mode, par, pending, mid);
                 else if (rows == 32) sor_block_launch<T, 1, 32>(c, cur, alt, dB, tabs, omega, tol, bnorm, l, check, ref_mode, par, pending);
                 else sor_block_launch<T, 1, 16>(c, cur, alt, dB, tabs, omega, tol, bnorm, l, check, ref_mode, par, pending);
@@ -2078,6 +2082,7 @@ int sor_sweeps(swm_ctx* c, void* dchi, void* dB, void* const* tabs, bool ref_mod
                                      c->stream));
         if (*host_done) return 0;
     }
+    const int npart = nblk + (seam ? 1 : 0);   // partial sums of a colour
     while (l <= max_sweeps && !*host_done) {
         const int64_t lend = std::min<int64_t>(max_sweeps, l + batch - 1);
         batch = std::min(2 * batch, batch_max);
@@ -2085,20 +2090,23 @@ int sor_sweeps(swm_ctx* c, void* dchi, void* dB, void* const* tabs, bool ref_mod
             const bool check = (l % every) == 0 || l == max_sweeps;
             for (int color = 0; color < 2; ++color) {
                 swm::SorArgs<T> a{};
-                a.Nx = c->Nx; a.Ny = c->Ny; a.P = c->P; a.color = color; a.sweep = (int)l;
+                a.Nx = c->Nx; a.Ny = c->Ny; a.P = c->P; a.color = color; a.sweep = (int)l; a.seam = seam;
                 a.chi = (T*)dchi; a.B = (const T*)dB; a.mask = c->mask;
                 a.relax = ref_mode ? (const double*)c->sor_relax : nullptr;
                 a.nrelax = c->sor_nrelax; a.omega = omega;
                 a.c1t = (const T*)tabs[0]; a.c3t = (const T*)tabs[1]; a.c4t = (const T*)tabs[2]; a.c5t = (const T*)tabs[3]; a.c5r = (const T*)tabs[4];
-                a.partial = c->sor_partial + color * nblk;
+                a.partial = c->sor_partial + color * npart;
                 a.done = c->sor_done;
                 a.residual_mode = ref_mode ? 0 : 1;
                 a.accumulate = check ? 1 : 0;
                 hipLaunchKernelGGL(swm::sor_sweep<T>, dim3(nblk), dim3(256), 0, c->stream, a);
+                if (!seam) continue;
+                a.partial += nblk;
+                hipLaunchKernelGGL(swm::sor_seam<T>, dim3(1), dim3(1024), 0, c->stream, a);
             }
             if (check)
                 hipLaunchKernelGGL(swm::sor_check, dim3(1), dim3(256), 0, c->stream, (const double*)c->sor_partial,
-                                   2 * nblk, (int)l, tol, bnorm, ref_mode ? 0 : 1, c->sor_done, c->sor_iters,
+                                   2 * npart, (int)l, tol, bnorm, ref_mode ? 0 : 1, c->sor_done, c->sor_iters,
                                    c->sor_norm);
         }
         HIPCHK(c, hipGetLastError());

@@ -2064,6 +2064,7 @@ march_kernel(const Dyn<T> d) {
 template <typename T>
 struct SorArgs {
     int Nx, Ny, P, color, sweep;
+    int seam;               // odd extents (bit 0 x, 1 y) of a grid whose colours do not alternate (sor_late)
     T* chi;
     const T* B;
     const uint8_t* mask;
@@ -2116,6 +2117,67 @@ __device__ __forceinline__ bool sor_test(const double* partial, int n, int sweep
     return *flag != 0;
 }
 
+// Across an open periodic seam of an odd extent the neighbours, columns 0 and
+// Nx - 1 (rows 0 and Ny - 1), have the same colour.  A sweep goes through its
+// cells in order of i and j, so column 0 is updated from the old column Nx - 1
+// and column Nx - 1 from the new column 0: the last column and row of such
+// extents come after a colour's other cells, their common corner after both.
+// (Updated with the others, with omega above 1.6 or so the pairs overshoot each
+// other and the sweeps diverge.)
+template <typename A>
+__device__ __forceinline__ int sor_late(const A& a, int i, int j) {
+    return ((a.seam & 1) && i == a.Nx - 1) + ((a.seam & 2) && j == a.Ny - 1);
+}
+
+// The update of cell (i, j); the square of its residual term, 0 on land.
+template <typename T>
+__device__ __forceinline__ double sor_cell(const SorArgs<T>& a, int i, int j) {
+    const size_t off = (size_t)j * a.P + i;
+    const uint8_t m = a.mask[off];
+    if (!(m & OC_E)) return 0.0;
+    const int ip = i + 1 == a.Nx ? 0 : i + 1, im = i == 0 ? a.Nx - 1 : i - 1;
+    const int jp = j + 1 == a.Ny ? 0 : j + 1, jm = j == 0 ? a.Ny - 1 : j - 1;
+    const uint8_t mip = a.mask[(size_t)j * a.P + ip], mjp = a.mask[(size_t)jp * a.P + i];
+    const int ouip = (mip >> 1) & 1, ou = (m >> 1) & 1, ovjp = (mjp >> 2) & 1, ov = (m >> 2) & 1;
+    const T c1 = ouip ? a.c1t[j] : T(0);
+    const T c2 = ou ? a.c1t[j] : T(0);
+    const T c3 = ovjp ? a.c3t[j] : T(0);
+    const T c4 = ov ? a.c4t[j] : T(0);
+    const int c5i = ((j * 3 + ouip + ou) * 2 + ovjp) * 2 + ov;
+    const T c5 = a.c5t[c5i];
+    T* chi = a.chi;
+    const T x = chi[off];
+    const T lhs = (((c1 * chi[(size_t)j * a.P + ip] + c2 * chi[(size_t)j * a.P + im]) +
+                    c3 * chi[(size_t)jp * a.P + i]) + c4 * chi[(size_t)jm * a.P + i]) + c5 * x;
+    const T r = lhs - a.B[off];
+    T res;
+    if (a.relax) {
+        int h = 2 * (a.sweep - 1) + a.color;
+        if (h >= a.nrelax) h = a.nrelax - 1;
+        res = dvr(T(a.relax[h]) * r, c5, a.c5r[c5i]);
+    } else {
+        res = dvr(T(a.omega) * r, c5, a.c5r[c5i]);
+    }
+    chi[off] = x - res;
+    const double q = a.residual_mode ? (double)r : (double)res;
+    return q * q;
+}
+
+// The sum of a block of NW wavefronts in fixed order, each wavefront's butterfly
+// then the wavefronts, to *out.
+template <int NW>
+__device__ __forceinline__ void sor_block_sum(double acc, double* red, double* out) {
+    for (int s = 32; s >= 1; s >>= 1) acc += __shfl_xor(acc, s, 64);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (lane == 0) red[wv] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = red[0];
+        for (int w = 1; w < NW; ++w) t += red[w];
+        *out = t;
+    }
+}
+
 // Each thread updates one cell of the colour; row j holds the colour's cells
 // at i = (j + colour + 1) % 2 + 2k (colour 0 = (i+j) even in 1-based indices).
 template <typename T>
@@ -2130,57 +2192,40 @@ __global__ void __launch_bounds__(256) sor_sweep(const SorArgs<T> a) {
     if (j < a.Ny) {
         // 1-based (i+j) even <=> 0-based (i+j) even
         const int i = 2 * kk + ((j + a.color) & 1);
-        if (i < a.Nx) {
-            const size_t off = (size_t)j * a.P + i;
-            const uint8_t m = a.mask[off];
-            if (m & OC_E) {
-                const int ip = i + 1 == a.Nx ? 0 : i + 1, im = i == 0 ? a.Nx - 1 : i - 1;
-                const int jp = j + 1 == a.Ny ? 0 : j + 1, jm = j == 0 ? a.Ny - 1 : j - 1;
-                const uint8_t mip = a.mask[(size_t)j * a.P + ip], mjp = a.mask[(size_t)jp * a.P + i];
-                const int ouip = (mip >> 1) & 1, ou = (m >> 1) & 1, ovjp = (mjp >> 2) & 1, ov = (m >> 2) & 1;
-                const T c1 = ouip ? a.c1t[j] : T(0);
-                const T c2 = ou ? a.c1t[j] : T(0);
-                const T c3 = ovjp ? a.c3t[j] : T(0);
-                const T c4 = ov ? a.c4t[j] : T(0);
-                const int c5i = ((j * 3 + ouip + ou) * 2 + ovjp) * 2 + ov;
-                const T c5 = a.c5t[c5i];
-                T* chi = a.chi;
-                const T x = chi[off];
-                const T lhs = (((c1 * chi[(size_t)j * a.P + ip] + c2 * chi[(size_t)j * a.P + im]) +
-                                c3 * chi[(size_t)jp * a.P + i]) + c4 * chi[(size_t)jm * a.P + i]) + c5 * x;
-                const T r = lhs - a.B[off];
-                T res;
-                if (a.relax) {
-                    int h = 2 * (a.sweep - 1) + a.color;
-                    if (h >= a.nrelax) h = a.nrelax - 1;
-                    res = dvr(T(a.relax[h]) * r, c5, a.c5r[c5i]);
-                } else {
-                    res = dvr(T(a.omega) * r, c5, a.c5r[c5i]);
-                }
-                chi[off] = x - res;
-                const double q = a.residual_mode ? (double)r : (double)res;
-                acc = q * q;
-            }
-        }
+        if (i < a.Nx && !sor_late(a, i, j)) acc = sor_cell(a, i, j);
     }
-    if (!a.accumulate) return;   // uniform: no barrier is skipped by part of the block
-    // fixed-order block reduction: wavefront butterfly then the 4 wave sums in order
-    for (int s = 32; s >= 1; s >>= 1) acc += __shfl_xor(acc, s, 64);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (lane == 0) red[wv] = acc;
+    if (a.accumulate) sor_block_sum<4>(acc, red, &a.partial[blockIdx.x]);   // uniform
+}
+
+// The colour's cells that sor_sweep leaves (sor_late), by one block: every other
+// cell of the last column and of the last row, then their corner.
+template <typename T>
+__global__ void __launch_bounds__(1024) sor_seam(const SorArgs<T> a) {
+    __shared__ double red[1024 / 64];
+    if (*a.done) return;
+    const int ic = a.Nx - 1, jr = a.Ny - 1;
+    const bool both = a.seam == 3;
+    double acc = 0.0;
+    if (a.seam & 1)
+        for (int j = 2 * threadIdx.x + ((ic + a.color) & 1); j < a.Ny - both; j += 2 * 1024) acc += sor_cell(a, ic, j);
+    if (a.seam & 2)
+        for (int i = 2 * threadIdx.x + ((jr + a.color) & 1); i < a.Nx - both; i += 2 * 1024) acc += sor_cell(a, i, jr);
     __syncthreads();
-    if (threadIdx.x == 0) a.partial[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
+    if (both && threadIdx.x == 0 && ((ic + jr) & 1) == a.color) acc += sor_cell(a, ic, jr);
+    if (a.accumulate) sor_block_sum<16>(acc, red, a.partial);
 }
 
 // K sweeps in one launch (fixed omega, or the reference's Chebyshev omega per
 // half sweep) on a TX x TY tile held in LDS, for the grids that sor_rows
 // (swm_sor.h) does not take: an odd extent with ocean faces across its
-// periodic seam, where the colours do not alternate.  2K-cell halo (read from
-// chi_in, written to chi_out: blocks read their halos while neighbours write).
-// Half sweep hs updates the colour-(hs % 2) cells at least hs + 1 cells inside
-// the staged block, whose dependency cones stay inside it, so the K sweeps give
-// each output cell exactly the values of K global red-black sweeps (sor_sweep,
-// same arithmetic).  With accumulate the last sweep's residuals of the output
+// periodic seam, where the colours do not alternate.  Halo of 2K + 2 cells (read
+// from chi_in, written to chi_out: blocks read their halos while neighbours
+// write).  Half sweep hs updates the colour-(hs % 2) cells at least hs + 1 cells
+// inside the staged block.  What is missing at its rim moves inwards by a cell
+// per half sweep, and by one more where it crosses the seam of an odd extent
+// (sor_late): once per extent of at least the halo's width, which the host
+// sees to.  So the K sweeps give each output cell exactly the values of K global
+// red-black sweeps (sor_sweep, same arithmetic).  With accumulate the last sweep's residuals of the output
 // cells (r, or the reference's res) are summed in FP64 in a fixed order into
 // partial[block]; block 0 first runs the previous launch's convergence test.
 //
@@ -2194,7 +2239,7 @@ __global__ void __launch_bounds__(256) sor_sweep(const SorArgs<T> a) {
 template <typename T, int TX, int TY, int K>
 __global__ void __launch_bounds__(256) sor_block(const SorArgs<T> a, const T* __restrict__ chi_in,
                                                  T* __restrict__ chi_out, int ntx) {
-    constexpr int H = 2 * K, W = TX + 2 * H, HH = TY + 2 * H, E = W * HH;
+    constexpr int H = 2 * K + 2, W = TX + 2 * H, HH = TY + 2 * H, E = W * HH;
     // per staged row: {0, c1}, {0, c3}, {0, c4}, c5[12], 1/c5[12]
     constexpr int TC1 = 0, TC3 = 2, TC4 = 4, TC5 = 6, TC5R = 18, NC = 30, NL = 27;
     static_assert(NL == 3 + 2 * 12 && NC == TC5R + 12, "row table layout");
@@ -2202,8 +2247,9 @@ __global__ void __launch_bounds__(256) sor_block(const SorArgs<T> a, const T* __
     __shared__ T s_B[E];
     __shared__ T s_c[HH][NC];
     // per cell: ov | ov(i,j+1) << 1 | (ou(i+1,j) + ou) << 2 | ou(i+1,j) << 4 | ou << 5 |
-    // ocean eta << 6 | colour ((i + j) % 2) << 7: the low four bits index c5
-    __shared__ uint8_t s_m[E];
+    // ocean eta << 6 | colour ((i + j) % 2) << 7 | sor_late << 8: the low four bits
+    // index c5
+    __shared__ uint16_t s_m[E];
     __shared__ double red[256 / 64];
     const int Nx = a.Nx, Ny = a.Ny, P = a.P;
     const int i0 = (blockIdx.x % ntx) * TX, j0 = (blockIdx.x / ntx) * TY;
@@ -2242,7 +2288,7 @@ __global__ void __launch_bounds__(256) sor_block(const SorArgs<T> a, const T* __
             const int mc = a.mask[off], mip = a.mask[(size_t)gj * P + gip], mjp = a.mask[(size_t)gjp * P + gi];
             const int ouip = (mip >> 1) & 1, ou = (mc >> 1) & 1, ovjp = (mjp >> 2) & 1, ov = (mc >> 2) & 1;
             rm[q] = ov | ovjp << 1 | (ouip + ou) << 2 | ouip << 4 | ou << 5 | ((mc & OC_E) ? 1 << 6 : 0) |
-                    ((gi + gj) & 1) << 7;
+                    ((gi + gj) & 1) << 7 | sor_late(a, gi, gj) << 8;
         }
     }
     // the 3 + 12 + 12 values of each staged row
@@ -2262,7 +2308,7 @@ __global__ void __launch_bounds__(256) sor_block(const SorArgs<T> a, const T* __
         if (e < E) {
             s_chi[e] = rchi[q];
             s_B[e] = rB[q];
-            s_m[e] = (uint8_t)rm[q];
+            s_m[e] = (uint16_t)rm[q];
         }
     }
 #pragma unroll
@@ -2277,12 +2323,12 @@ __global__ void __launch_bounds__(256) sor_block(const SorArgs<T> a, const T* __
     __syncthreads();
     // Without an odd periodic wrap inside the block the colours alternate
     // along every staged row (colour = (p0 + lx + ly) % 2): each half-sweep
-    // then visits only the cells of its colour; otherwise it walks the block
-    // and tests the colour bit.
+    // then visits only the cells of its colour; otherwise it finds them by their
+    // codes.
     static_assert(W % 2 == 0, "pairs of cells along a row");
     const bool regular = ((Nx & 1) == 0 || (i0 - H >= 0 && i0 - H + W <= Nx)) &&
                          ((Ny & 1) == 0 || (j0 - H >= 0 && j0 - H + HH <= Ny));
-    const int p0 = (i0 + j0) & 1;
+    const int p0 = (i0 + j0) & 1, nlate = (a.seam & 1) + (a.seam >> 1);
     double acc = 0.0, acc_mid[3] = {0.0, 0.0, 0.0};
     // the update of cell (lx, ly) (sor_sweep's arithmetic): its new value, and
     // the residual term r or res; land cells keep their value
@@ -2317,22 +2363,32 @@ __global__ void __launch_bounds__(256) sor_block(const SorArgs<T> a, const T* __
         }
     };
     constexpr int NIM = (HH * (W / 2) + 255) / 256;   // cells of one colour per thread, at most
+    // omega of half sweep hs: the reference's Chebyshev schedule (held once
+    // stationary) or the fixed omega; a.sweep is the launch's first sweep
+    auto omega = [&](int hs) {
+        if (!a.relax) return T(a.omega);
+        const int h = 2 * (a.sweep - 1) + hs;
+        return T(a.relax[h < a.nrelax ? h : a.nrelax - 1]);
+    };
+    // a cell's new value and its residual, where half sweep hs is tested: the
+    // launch's last sweep, and with mid the earlier ones
+    auto put = [&](int hs, int lx, int ly, T nv, T rq) {
+        s_chi[ly * W + lx] = nv;
+        const int sw = hs / 2;
+        if (a.accumulate && sw == K - 1) add(acc, lx, ly, rq);
+        if (a.mid && sw < K - 1) add(acc_mid[sw < 3 ? sw : 0], lx, ly, rq);
+    };
+    auto end = [&](int hs) {
+        __syncthreads();
+        if (!(hs & 1) || !a.mid || hs / 2 >= K - 1) return;   // uniform
+        store_out(a.chi_mid[hs / 2 < 3 ? hs / 2 : 0]);        // chi after a sweep, before the next one changes it
+        __syncthreads();
+    };
+    if (regular) {
 #pragma unroll
-    for (int hs = 0; hs < 2 * K; ++hs) {
-        const int color = hs & 1;
-        const int lo = hs + 1;
-        const bool tail = a.accumulate && hs >= 2 * K - 2;
-        const int sw = hs / 2;                          // the sweep of this half sweep
-        const bool inner = a.mid && sw < K - 1;         // an earlier sweep, tested too (mid)
-        // omega of this half-sweep: the reference's Chebyshev schedule (held
-        // once stationary) or the fixed omega; a.sweep is the launch's first sweep
-        T om = T(a.omega);
-        if (a.relax) {
-            int h = 2 * (a.sweep - 1) + hs;
-            if (h >= a.nrelax) h = a.nrelax - 1;
-            om = T(a.relax[h]);
-        }
-        if (regular) {
+        for (int hs = 0; hs < 2 * K; ++hs) {
+            const int color = hs & 1, lo = hs + 1;
+            const T om = omega(hs);
             // rows lo .. HH-1-lo, (W - 2 lo) / 2 cells of the colour in each
             const int RW2 = (W - 2 * lo) / 2, n = (HH - 2 * lo) * RW2;
             T nv[NIM], rq[NIM];
@@ -2352,30 +2408,41 @@ __global__ void __launch_bounds__(256) sor_block(const SorArgs<T> a, const T* __
                 oc[k] = upd(lxs[k], lys[k], om, nv[k], rq[k]) && tid + k * 256 < n;
             }
 #pragma unroll
-            for (int k = 0; k < NIM; ++k) {
-                if (k * 256 < n && oc[k]) {
-                    s_chi[lys[k] * W + lxs[k]] = nv[k];
-                    if (tail) add(acc, lxs[k], lys[k], rq[k]);
-                    if (inner) add(acc_mid[sw < 3 ? sw : 0], lxs[k], lys[k], rq[k]);
-                }
-            }
-        } else {
-            for (int q = tid; q < E; q += 256) {
-                const int lx = q % W, ly = q / W;
-                if (lx < lo || lx > W - 1 - lo || ly < lo || ly > HH - 1 - lo) continue;
-                if ((s_m[q] >> 7) != color) continue;
-                T nv, rq;
-                if (upd(lx, ly, om, nv, rq)) {
-                    s_chi[q] = nv;
-                    if (tail) add(acc, lx, ly, rq);
-                    if (inner) add(acc_mid[sw < 3 ? sw : 0], lx, ly, rq);
-                }
-            }
+            for (int k = 0; k < NIM; ++k)
+                if (k * 256 < n && oc[k]) put(hs, lxs[k], lys[k], nv[k], rq[k]);
+            end(hs);
         }
-        __syncthreads();
-        if ((hs & 1) && inner) {   // chi after sweep sw, before the next sweep changes it
-            store_out(a.chi_mid[sw < 3 ? sw : 0]);
-            __syncthreads();
+    } else {
+        // Two neighbours along a row hold one cell to update, or none: across the
+        // seam they have the same colour, but one of them comes later.
+#pragma unroll
+        for (int hs = 0; hs < 2 * K; ++hs) {
+            const int lo = hs + 1, RW2 = (W - 2 * lo) / 2, n = (HH - 2 * lo) * RW2;
+            const T om = omega(hs);
+#pragma unroll 1
+            for (int late = 0; late <= nlate; ++late) {   // sor_late's order
+                if (late) __syncthreads();
+                const int want = (hs & 1) | late << 1;
+                T nv[NIM], rq[NIM];
+                int lxs[NIM], lys[NIM];
+                bool oc[NIM];
+#pragma unroll
+                for (int k = 0; k < NIM; ++k) {
+                    oc[k] = false;
+                    if (k * 256 >= n) continue;
+                    const int q = tid + k * 256 < n ? tid + k * 256 : n - 1;
+                    const int ly = lo + q / RW2, lx = lo + 2 * (q % RW2), e = ly * W + lx;
+                    const bool m0 = s_m[e] >> 7 == want, m1 = s_m[e + 1] >> 7 == want;
+                    lys[k] = ly;
+                    lxs[k] = m0 ? lx : lx + 1;
+                    if (late && !(m0 || m1)) continue;
+                    oc[k] = upd(lxs[k], ly, om, nv[k], rq[k]) && (m0 || m1) && tid + k * 256 < n;
+                }
+#pragma unroll
+                for (int k = 0; k < NIM; ++k)
+                    if (k * 256 < n && oc[k]) put(hs, lxs[k], lys[k], nv[k], rq[k]);
+            }
+            end(hs);
         }
     }
     store_out(chi_out);
