@@ -585,26 +585,16 @@ __device__ __forceinline__ void tile_load(const Dyn<T>& d, const int t, RG& R, c
     constexpr int EW = TX + 2;
     constexpr int EH = TY + 2;
     constexpr int E = EW * EH;
-    constexpr int NO = (TX * TY + NT - 1) / NT;
-    constexpr int NTR = NTRC > 0 ? NTRC : 1;
     CStatics<T>& a = *(CStatics<T>*)d.s;
     const int i0 = (t % d.ntx) * TX;
     const int j0 = (t / d.ntx) * TY;
     const int Nx = a.Nx, Ny = a.Ny, P = a.P;
-    const bool FN = (VAR == VAR_FN);
     // planes of this step's roles
     T* const st = d.state;
     const long long pl = d.plane;
-    const int r0 = d.ring, r1 = d.ring == 2 ? 0 : d.ring + 1, r2 = d.ring == 0 ? 2 : d.ring - 1;
     const T* const su = st + (PL_U + d.cur) * pl;
     const T* const sv = st + (PL_V + d.cur) * pl;
     const T* const se = st + (PL_E + d.cur) * pl;
-    const T* const Gu1 = st + (PL_GU + r0) * pl;
-    const T* const Gu2 = st + (PL_GU + r1) * pl;
-    const T* const Gv1 = st + (PL_GV + r0) * pl;
-    const T* const Gv2 = st + (PL_GV + r1) * pl;
-    const T* const Ge1 = st + (PL_GE + r0) * pl;
-    const T* const Ge2 = st + (PL_GE + r1) * pl;
 
     if (HIST) tile_load_hist<T, VAR, NTRC, TX, TY, DIAG>(d, t, R, tid);
 
@@ -696,8 +686,6 @@ __device__ __forceinline__ void tile_stage(const Dyn<T>& d, const int t, const R
     constexpr int EW = TX + 2;
     constexpr int EH = TY + 2;
     constexpr int E = EW * EH;
-    constexpr int NO = (TX * TY + NT - 1) / NT;
-    constexpr int NTR = NTRC > 0 ? NTRC : 1;
     T* const s_u = lds.u;
     T* const s_v = lds.v;
     T* const s_eta = lds.Ed;
@@ -707,23 +695,9 @@ __device__ __forceinline__ void tile_stage(const Dyn<T>& d, const int t, const R
     uint16_t* const s_m = lds.m;
 
     CStatics<T>& a = *(CStatics<T>*)d.s;
-    const int i0 = (t % d.ntx) * TX;
     const int j0 = (t / d.ntx) * TY;
-    const int Nx = a.Nx, Ny = a.Ny, P = a.P;
+    const int Ny = a.Ny;
     const bool FN = (VAR == VAR_FN);
-    // planes of this step's roles
-    T* const st = d.state;
-    const long long pl = d.plane;
-    const int r0 = d.ring, r1 = d.ring == 2 ? 0 : d.ring + 1, r2 = d.ring == 0 ? 2 : d.ring - 1;
-    const T* const su = st + (PL_U + d.cur) * pl;
-    const T* const sv = st + (PL_V + d.cur) * pl;
-    const T* const se = st + (PL_E + d.cur) * pl;
-    const T* const Gu1 = st + (PL_GU + r0) * pl;
-    const T* const Gu2 = st + (PL_GU + r1) * pl;
-    const T* const Gv1 = st + (PL_GV + r0) * pl;
-    const T* const Gv2 = st + (PL_GV + r1) * pl;
-    const T* const Ge1 = st + (PL_GE + r0) * pl;
-    const T* const Ge2 = st + (PL_GE + r1) * pl;
 
     constexpr int NE = (E + NT - 1) / NT;
     const auto& rm = R.m;
