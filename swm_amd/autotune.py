@@ -12,9 +12,11 @@ Search spaces (every candidate gives the same results bit for bit):
   persistent grid draining per-XCD tile queues) - swm_gpu_batch_tune, likewise;
 * the fixed-omega SOR: halo width of the blocked sweeps (0 = one launch per
   colour; 2, 4, 8 cells = 1, 2, 4 sweeps per launch, each sweep consuming two
-  halo cells) x convergence-test cadence (1..16 sweeps) x rows of the 64-wide
-  LDS tile (16 or 32: fewer halo cells per output, more LDS), where the sweeps
-  per launch must divide the cadence and the 8-cell halo takes 16-row tiles.
+  halo cells; -1 = the library's choice, four whatever the cadence) x
+  convergence-test cadence (1..16 sweeps), where a set halo's sweeps per launch
+  must divide the cadence; on grids open across the periodic seam of an odd
+  extent also x rows of the 64-wide LDS tile (16 or 32: fewer halo cells per
+  output, more LDS; the 8-cell halo takes 16-row tiles).
   The candidates are raced by successive halving:
   every survivor solves the same right-hand side from the same zero start for
   a fixed number of sweeps (tolerance 0, so none stops early); the slower half
@@ -32,6 +34,8 @@ import json
 import os
 import time
 from typing import Iterable, Optional, Sequence
+
+import numpy as np
 
 from . import gpu
 
@@ -115,13 +119,39 @@ def tune_batch(b: "gpu.SwmBatch", steps: int = 10, cache: Optional[TuneCache] = 
     return dict(res, cached=False)
 
 
-def sor_candidates(halos: Iterable[int] = (0, 2, 4, 8), cadences: Iterable[int] = (1, 2, 4, 8, 16),
+def sor_candidates(halos: Iterable[int] = (-1, 0, 2, 4, 8), cadences: Iterable[int] = (1, 2, 4, 8, 16),
                    rows: Iterable[int] = (16, 32)):
     """(halo, cadence, rows) whose sweeps per launch (halo / 2) divide the
-    cadence; 32-row tiles only for blocked sweeps of at most 2 per launch (the
-    unblocked colour launches have no tile)."""
+    cadence; halo -1 is the library's own choice, which fits every cadence.  The
+    taller tiles only for blocked sweeps of at most 2 per launch (the unblocked
+    colour launches have no tile)."""
     return [(h, c, r) for h in halos for c in cadences for r in rows
             if (h <= 2 or c % (h // 2) == 0) and (r == 16 or 0 < h <= 4)]
+
+
+def colours_alternate(s) -> bool:
+    """Whether the sweeps run on register tiles: even extents, or odd ones with
+    no ocean face across their periodic seam (every closed basin)."""
+    return ((s.Nx % 2 == 0 or not np.any(s.grids["u"].ocean[:, 0])) and
+            (s.Ny % 2 == 0 or not np.any(s.grids["v"].ocean[0])))
+
+
+def sor_sweeps_per_launch(s, halo: int, cadence: int) -> int:
+    """The sweeps that go to a launch of a fixed-omega solve (0: one colour)."""
+    if halo >= 0:
+        return halo // 2
+    return 4 if colours_alternate(s) else 2 - cadence % 2
+
+
+def distinct_sor_candidates(s, candidates):
+    """Of the candidates that run the same code on the domain s, the first:
+    register tiles take their height from the grid whatever rows says, and the
+    library's own halo is one of the others."""
+    out = {}
+    for h, c, r in candidates:
+        k = sor_sweeps_per_launch(s, h, c)
+        out.setdefault((k, c, 0 if colours_alternate(s) or k == 0 else r), (h, c, r))
+    return list(out.values())
 
 
 def apply_sor(m: "gpu.SwmGpu", halo: int, cadence: int, rows: int = 16):
@@ -132,17 +162,17 @@ def apply_sor(m: "gpu.SwmGpu", halo: int, cadence: int, rows: int = 16):
 
 
 def tune_sor(m: "gpu.SwmGpu", omega: float = 1.9, fp32_sweeps: bool = False,
-             halos: Sequence[int] = (0, 2, 4, 8), cadences: Sequence[int] = (1, 2, 4, 8, 16),
+             halos: Sequence[int] = (-1, 0, 2, 4, 8), cadences: Sequence[int] = (1, 2, 4, 8, 16),
              rows: Sequence[int] = (16, 32), sweeps: int = 64, cache: Optional[TuneCache] = None) -> dict:
-    """Successive halving over (halo, cadence, rows): time `sweeps`
-    fixed-omega sweeps of every candidate, keep the faster half, double the
+    """Successive halving over (halo, cadence, rows), each kind of launch once: time
+    `sweeps` fixed-omega sweeps of every candidate, keep the faster half, double the
     sweeps, until one is left; applies and returns it."""
     key = f"{signature(m)}/w{omega}/f{int(bool(fp32_sweeps))}"
     hit = cache.get("sor", key) if cache else None
     if hit is not None:
         apply_sor(m, hit["halo"], hit["check_every"], hit.get("rows", 16))
         return dict(hit, cached=True)
-    cand = sor_candidates(halos, cadences, rows)
+    cand = distinct_sor_candidates(m.s, sor_candidates(halos, cadences, rows))
     rounds = []
     n = sweeps
     while len(cand) > 1:
@@ -158,7 +188,7 @@ def tune_sor(m: "gpu.SwmGpu", omega: float = 1.9, fp32_sweeps: bool = False,
         n *= 2
     (h, c, r), = cand
     apply_sor(m, h, c, r)
-    res = {"halo": h, "check_every": c, "rows": r, "sweeps_per_launch": h // 2, "rounds": rounds}
+    res = {"halo": h, "check_every": c, "rows": r, "sweeps_per_launch": sor_sweeps_per_launch(m.s, h, c), "rounds": rounds}
     if cache:
         cache.put("sor", key, res)
     return dict(res, cached=False)

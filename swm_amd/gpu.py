@@ -417,12 +417,13 @@ class SwmGpu:
         self._check(self.L.swm_gpu_set_sor_check_every(self._h, int(every)), "swm_gpu_set_sor_check_every")
 
     def set_sor_halo(self, halo: int):
-        """LDS halo of the blocked fixed-omega SOR sweeps in cells (2 x sweeps
-        per launch: 2, 4, 8; 0 = one launch per colour; -1 = from the cadence)."""
+        """Halo of the blocked SOR sweeps in cells (2 x sweeps per launch: 2, 4, 8;
+        0 = one launch per colour; -1 = the library's choice, four sweeps)."""
         self._check(self.L.swm_gpu_set_sor_halo(self._h, int(halo)), "swm_gpu_set_sor_halo")
 
     def set_sor_tile_rows(self, rows: int):
-        """Rows of the blocked SOR sweeps' 64-column tile (16 or 32)."""
+        """Rows of the 64-column tile of SOR sweeps on grids open across the
+        periodic seam of an odd extent (16 or 32)."""
         self._check(self.L.swm_gpu_set_sor_tile_rows(self._h, int(rows)), "swm_gpu_set_sor_tile_rows")
 
     def set_launch_mode(self, graphs: bool):
