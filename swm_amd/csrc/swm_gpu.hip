@@ -956,14 +956,17 @@ Dyn<T> make_dyn(swm_ctx* c, int tile) {
 }
 
 // FULLY_NONLINEAR FP64 domains of more tiles than this split off the all-ocean
-// ones (step_kernel_split): two rounds of the 1280 blocks that are resident at
-// once.  Below, a step is mostly one tile's latency and the longer kernel costs 2
-// to 4 % of it (200^2: 5.50 -> 5.61 us, 512^2 the same); above, it saves mask
-// arithmetic: 1024x768 40.9 -> 40.5 us, 1024^2 with 5 % land and a tracer 38.7 ->
-// 38.1, with no land and two 45.4 -> 42.3, 2304x1800 122.5 -> 116.4, 4096x2048 329
-// -> 316.  FP64 batches take the same line (batch_kernel_split): 14 members of 8856
-// tiles 92.0 -> 87.8 us a step, 30 of 34165 315 -> 299, 40 small ones of 5530 the
-// same within 1 %; below it the split cost 4 members of 163 tiles 1.4 %.
+// ones (step_kernel_split): with a tracer, five blocks on each of 256 CUs, it is two
+// rounds of resident blocks.  Below, a step is mostly one tile's latency and the
+// longer kernel costs 2 to 4 % of it (200^2: 5.50 -> 5.61 us); above, it saves mask
+// arithmetic.  us a step without -> with the split, for no, one and two tracers:
+// 640x800 (2000 tiles) 17.15 -> 17.50, 22.35 -> 21.57, 24.9 -> 23.9; 768x900 (2712)
+// 20.95 -> 20.81, 28.4 -> 26.7, 31.2 -> 29.3; 1024x768 (3072) 22.6 -> 22.65, 30.4 ->
+// 29.4, 34.1 -> 33.5; 2304x1800 without tracers 122.5 -> 116.4, 4096x2048 329 -> 316.
+// (With tracers the line could lie lower.)  FP64 batches take it too
+// (batch_kernel_split): 14 members of 8856 tiles 92.0 -> 87.8 us a step, 30 of 34165
+// 315 -> 299, 40 small ones of 5530 the same within 1 %; below it the split cost 4
+// members of 163 tiles 1.4 %.
 constexpr int kSplitTiles = 2560;
 
 template <typename T, int TX, int TY, bool DIAG, bool LATE = false>
@@ -1400,26 +1403,11 @@ static int create_impl(swm_ctx* c, const swm_desc* d) {
         c->mask = (uint8_t*)dalloc(c, m.size());
         if (!c->mask) return fail(c, "out of device memory", 3);
         HIPCHK(c, copy_sync(c, c->mask, m.data(), m.size(), hipMemcpyHostToDevice));
-        // per-cell codes: the cell's masks and its neighbours'
-        std::vector<uint16_t> cc((size_t)c->Ny * c->P, 0);
-        const int Nx = c->Nx, Ny = c->Ny;
-        for (int j = 0; j < Ny; ++j) {
-            const uint8_t *r = &m[(size_t)j * c->P], *rs = &m[(size_t)(j ? j - 1 : Ny - 1) * c->P],
-                          *rn = &m[(size_t)(j + 1 < Ny ? j + 1 : 0) * c->P];
-            for (int i = 0; i < Nx; ++i) {
-                const int w = i ? i - 1 : Nx - 1, e = i + 1 < Nx ? i + 1 : 0;
-                auto bit = [](uint8_t x, uint8_t oc, int at) { return x & oc ? 1 << at : 0; };
-                cc[(size_t)j * c->P + i] = (uint16_t)(
-                    r[i] | bit(r[w], swm::OC_E, swm::CC_EW) | bit(rs[i], swm::OC_E, swm::CC_ES) |
-                    bit(rs[w], swm::OC_E, swm::CC_ESW) | bit(rs[i], swm::OC_U, swm::CC_US) |
-                    bit(r[w], swm::OC_V, swm::CC_VW) | bit(rn[i], swm::OC_V, swm::CC_VN) |
-                    bit(r[e], swm::OC_U, swm::CC_UE) | bit(r[e], swm::OC_E, swm::CC_EE) |
-                    bit(rn[i], swm::OC_E, swm::CC_EN) | bit(rn[i], swm::OC_H, swm::CC_HN));
-            }
-        }
-        c->code = (uint16_t*)dalloc(c, cc.size() * sizeof(uint16_t));
+        c->code = (uint16_t*)dalloc(c, m.size() * sizeof(uint16_t));
         if (!c->code) return fail(c, "out of device memory", 3);
-        HIPCHK(c, copy_sync(c, c->code, cc.data(), cc.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+        hipLaunchKernelGGL(swm::step_code_kernel, dim3((unsigned)((m.size() + 255) / 256)), dim3(256), 0, c->stream,
+                           c->Nx, c->Ny, c->P, c->mask, c->code);
+        HIPCHK(c, hipGetLastError());
     }
     const int8_t *mu = c->hmask[1].data(), *mv = c->hmask[2].data(), *me = c->hmask[3].data();
     int rc = 0;
