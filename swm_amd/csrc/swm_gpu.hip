@@ -1819,11 +1819,11 @@ int sor_rows_prepare(swm_ctx* c) {
 }
 
 // Tile heights of sor_rows (wavefronts x rows each).  A launch's time is its
-// slowest block's, so a grid takes the smallest tile of which every CU gets at
-// most one (32 rows: 10.1 us a launch against 13.2 with 48 and 15.0 with 64 at
-// 720 x 361 FP64; 64 rows: 10.7 against 12.2 and 13.0 at 1201 x 800 FP32);
-// larger grids take 48 rows, of which a CU holds two, so that one loads while
-// the other sweeps (26.2 against 29.7 with 64 rows at 2048 x 1024 FP64).
+// slowest block's, so a grid takes the smallest tile of which every CU gets at most
+// one (timed on the host: 32 rows 10.1 us a launch against 13.2 with 48 and 15.0
+// with 64 at 720 x 361 FP64; 64 rows: 10.7 against 12.2 and 13.0 at 1201 x 800
+// FP32); larger grids take 48 rows, of which a CU holds two, so that one loads
+// while the other sweeps (26.2 against 29.7 with 64 rows at 2048 x 1024 FP64).
 int sor_tile_height(const swm_ctx* c, int H) {
     auto tiles = [&](int hh) {
         return (long)((c->Nx + 127 - 2 * H) / (128 - 2 * H)) * ((c->Ny + hh - 2 * H - 1) / (hh - 2 * H));

@@ -187,14 +187,14 @@ __device__ __forceinline__ void pairs(F&& f) {
 // inside it are exactly those of global red-black sweeps, operation by
 // operation those of sor_sweep.
 //
-// Bound: vector issue of the sweeps (22 instructions a cell where every
-// neighbour is ocean, 18 of them FP64 at 4 cycles; 40 where a wavefront holds
+// Bound: vector issue of the sweeps (23 instructions a cell where every
+// neighbour is ocean, 18 of them FP64 at 4 cycles; 41 where a wavefront holds
 // land, whose coefficients are masked lane by lane) and, a third of a launch,
 // the tile's loads, which nothing overlaps when a CU has one block.  The LDS
 // tiles of sor_block spend about 130 instructions a cell and sweep on
-// addresses, masks and LDS traffic.  Four sweeps a launch, us per launch,
-// LDS tiles -> here: 51.6 -> 26.2 at 2048 x 1024 FP64, 33.6 -> 10.7 at
-// 1201 x 800 FP32, 36.4 -> 10.1 at 720 x 361 FP64 (reference mode).
+// addresses, masks and LDS traffic.  Four sweeps a launch, us per launch in the
+// kernel trace, LDS tiles -> here: 51.6 -> 27.1 at 2048 x 1024 FP64, 33.6 -> 11.2
+// at 1201 x 800 FP32, 36.4 -> 12.0 at 720 x 361 FP64 (reference mode).
 template <typename T, int NW, int R>
 __global__ void __launch_bounds__(NW * 64)
 sor_rows(const SorRowsArgs<T> a, const T* __restrict__ chi_in, T* __restrict__ chi_out) {
